@@ -39,6 +39,8 @@
 // linearity: y = inv_rms * (x (1 + gamma)) W, so its sum of squares comes
 // from the same x loads and the factor scales the column sums.
 #include "qm_device.h"
+#include "qm_q4_tiles.h"
+#include <type_traits>
 #include "qm_kernel_args.h"
 
 #define Q4_THREADS 512
@@ -412,20 +414,54 @@ extern "C" __global__ __launch_bounds__(256) void qm_q4_repack(Q4RepackArgs A) {
 // Prefill: C[m][n] = X[m][k] W on MFMA (gemm_q4, gemv.rs:529-542, for
 // seq_len > 1).  X is f16 (qm_rms_norm_f16 produces it from the f32 hidden
 // state, fusing the layer's RMSNorm) or bf16 (the mixer outputs and the
-// MLP's silu(g) * u).  W stays Q4 in HBM and is dequantized on its way into
-// LDS: s * (q - 8) rounded once to f16 and, for a bf16 X, on to bf16.  An
-// f16 X runs v_mfma_f32_16x16x32_f16; a bf16 X is staged as it is and runs
-// v_mfma_f32_16x16x32_bf16, so it keeps fp32's range.
-// Workgroup tile 128 x 256, four waves of 64 x 128 (4 x 8 MFMA tiles: 12
-// fragment reads feed 32 MFMAs), k steps of 32 in two LDS stages with one
-// barrier per step.  LDS rows are k-contiguous, X as [m][k] and W as [n][k],
-// padded to 40 halves (80 bytes) so the 16 rows of a fragment read land in
-// 16 distinct bank slots; a lane's A operand (row m, k 8kg .. +7) and B
-// operand (column n, k 8kg .. +7) are then one 16-byte read each.
+// MLP's silu(g) * u).  W stays Q4 in HBM and in LDS and is dequantized into
+// the MFMA operand registers: s * (q - 8) rounded once to f16 and, for a bf16
+// X, on to bf16.  An f16 X runs v_mfma_f32_16x16x32_f16; a bf16 X is used as
+// it is and runs v_mfma_f32_16x16x32_bf16, so it keeps fp32's range.
+//
+// Operand form.  A wave computes 16 MI rows x 16 NJ columns, and lane
+// fr = lane & 15 of its fragment j holds column NJ fr + j.  The codes a lane
+// needs of one row of k are then NJ neighbouring nibbles of one code word,
+// and its outputs are NJ neighbouring columns, stored straight from the
+// accumulators (16 bytes of fp32 at NJ = 4).
+//
+// Staging.  64 rows of k are a stage: x rows, raw codes and scales are copied
+// to LDS by DMA, no registers and no LDS store instructions, each instruction
+// covering whole 128-byte lines (an x operand read straight from global
+// memory has 16 rows in 16 neighbouring lanes, which the memory path takes
+// one lane at a time: measured 60 cache accesses per load instruction, the L1
+// at one access per cycle the whole launch).  16-byte chunks are xor-swizzled
+// in each row or tile so that the operand reads meet no bank conflict
+// (SQ_LDS_BANK_CONFLICT 0).  One barrier per stage.
+//
+// What bounds it.  Large m: issue slots.  Per step of 32 rows a 128 x 64 wave
+// tile issues 32 MFMAs and ~80 VALU instructions (1.75 per weight pair and
+// addressing), and a probe shows two VALU instructions per 16-cycle MFMA are
+// free and each further one costs four cycles; timing copies put the
+// dequantization at 28 us and the DMA at 28 us of 160 us (4096 x 2560 x
+// 8192), without both and the barrier 109 us, which is what the MFMAs alone
+// take.  Few rows: the chain of stages, ~0.45 us each for the smallest tile;
+// so k is split over the waves of a workgroup (WK groups, their partial tiles
+// added in group order through LDS at the end) until there is a workgroup
+// for every CU.
+//
+// Measured against the form it replaces (codes dequantized once per
+// workgroup into LDS, 128 x 256 tiles, one barrier per 32 rows), us, same
+// box, rotating weights:
+//   m x k x n            before    now
+//   45 x 2560 x 8192       39.1    8.1     (DeltaNet in_proj_qkv)
+//   45 x 9216 x 2560      141.9   14.4     (down_proj, bf16 x)
+//   300 x 9216 x 2560     141     36
+//   700 x 4096 x 2560      64     28       (o_proj, bf16 x)
+//   4096 x 2560 x 8192    187    152       (1.13 PFLOP/s)
+//   4096 x 9216 x 2560    271    238
+//   4096 x 2560 x 32        9.9    5.6     (in_proj_a / b)
+//   4096 x 2560 x 9216 gate/up  406    337  (1.15 PFLOP/s)
+// Tried and no faster: dequantizing the next step's operand between the
+// MFMAs of this one (explicit interleave; 0-3% either way), two LDS stages
+// instead of three (0-2%), and reading x and codes without LDS (3-4 x slower
+// from 300 rows on, for the access count above).
 // ---------------------------------------------------------------------------
-#define GM_TK 32
-#define GM_LDK 40
-
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -439,302 +475,298 @@ __device__ __forceinline__ uint32_t f16x2_to_bf16x2(half2 h) {
     return __builtin_bit_cast(uint32_t, b);
 }
 
-// XBF16: x is bf16 and W is rounded on to bf16 (bf16 MFMA); else both f16.
-// GU: the gate/up form.  The workgroup's 256 W rows of LDS are then
-// 16-column fragments of the gate and up weights alternately, over 128
-// output columns, so a wave's fragments j (gate) and j + 1 (up) hold the
-// same outputs and the epilogue writes silu(g) * u as bf16 (whose range,
-// unlike f16's, holds any product of the fp32 accumulators).
-// A workgroup is WM x WN waves; a wave computes MI x NJ MFMA tiles of
-// 16 x 16 (16 MI rows, 16 NJ columns), so the workgroup tile is TM x TN =
-// 16 MI WM x 16 NJ WN.  128 x 256 (2 x 2 waves of 64 x 128) where there are
-// tiles enough for two workgroups per CU; for narrow outputs that would
-// leave CUs idle, 128 x 128 (n = 2560: 10 column tiles of 256) or 64 x 128
-// (n = 1024); n = 32 has a kernel of its own below.  The W tile is staged by
-// threads 0 .. TN-1.  (64 x 256 tiles, four waves of 64 x 64 side by side,
-// measured 2% slower on the 4096-token prefill.)
-template <bool XBF16, bool GU, int WM, int WN, int MI, int NJ>
-__device__ __forceinline__ void q4_gemm_body(const Q4GemmArgs& A) {
-    constexpr int TM = 16 * MI * WM, TN = 16 * NJ * WN, NTH = 64 * WM * WN;
-    static_assert(!GU || (WN == 2 && NJ == 8), "the gate/up form pairs fragments j, j + 1 over 256 LDS rows");
-    static_assert(NTH >= TN && (TM * GM_TK / NTH == 8 || TM * GM_TK / NTH == 16), "staging shape");
-    __shared__ __attribute__((aligned(16))) _Float16 sA[2][TM][GM_LDK];
-    __shared__ __attribute__((aligned(16))) _Float16 sB[2][TN][GM_LDK];
-    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-    constexpr int NCOLS = GU ? TN / 2 : TN;              // output columns per workgroup
-    const int nbn = (A.n + NCOLS - 1) / NCOLS;
-    // consecutive workgroups walk n within one row block: the row block's X
-    // (k x TM halves) is reused from L2 across its column tiles
-    const int bm = (int)blockIdx.x / nbn, bn = (int)blockIdx.x % nbn;
-    const int m0 = bm * TM, n0 = bn * NCOLS;
-    const int wm = w / WN, wn = w % WN;
-    const int T = A.tile, K = A.k;
-    const int nk = K / GM_TK;
+// LDS of one k-group and stage: x rows [16 MI][64] (chunk c of row r at slot
+// c ^ (r & 7)), then per wave the codes of its 16 NJ columns x 64 rows and
+// its scales [NJ / 2][64] (256 bytes).
+template <int MI, int NJ, int WN, int WK, int NST>
+struct Q4GemmLds {
+    static constexpr int X = 16 * MI * 128, C = 512 * NJ, S = 256;
+    static constexpr int STAGE = X + WN * (C + S);
+    static constexpr int BYTES = WK * NST * STAGE;
+};
 
-    // X staging: thread -> row tid / (32 / XH), XH halves of k
-    constexpr int XH = TM * GM_TK / NTH;                 // 16 or 8 halves per thread
-    const int ar = tid / (32 / XH), ah = tid % (32 / XH);
-    const uint16_t* xrow = A.x + (size_t)min(m0 + ar, A.m - 1) * K + XH * ah;
-    // W staging: thread -> 8-column block c8 of the tile and RQ rows
-    // RQ rq .. +RQ-1 of the step, with every thread taking a share (RQ = 4
-    // when the tile has as many columns as the workgroup threads, else 2); a
-    // block is 4 code bytes of one row (T = 16: half of a tile row, T = 8: a
-    // whole one)
-    constexpr int RQ = NTH == TN ? 4 : 2;
-    const int c8 = tid / (32 / RQ), rq = tid % (32 / RQ);
-    // GU: LDS rows 8 c8 .. +7 are half of fragment c8 / 2, of the up weight
-    // when that fragment is odd
-    const bool up = GU && ((c8 >> 1) & 1);
-    const int ccol = GU ? 16 * (c8 >> 2) + 8 * (c8 & 1) : 8 * c8;
-    const int ncl = min(n0 + ccol, A.n - 8);            // valid block for loads
-    const size_t cstride = (size_t)(T / 2);
-    const uint8_t* bcodes = (up ? A.codes2 : A.codes) + (size_t)(ncl / T) * K * cstride + (ncl % T) / 2 +
-                            RQ * rq * cstride;
-    const uint16_t* bsc = (up ? A.gscales2 : A.gscales) + (size_t)(ncl / 32) * K + RQ * rq;
-    const bool wthread = NTH * RQ == 4 * TN || tid < TN * 4 / RQ;
+// BIG: 64-bit lane offsets (k above QM_Q4_GEMM_MAX_K32).
+template <bool XBF16, bool GU, int MI, int NJ, int WN, int WK, int NST, int T, bool BIG>
+__device__ __forceinline__ void q4_gemm_loop(const Q4GemmArgs& A, int m0, int n0, char* smem, floatx4 (&acc)[MI][NJ]) {
+    using L = Q4GemmLds<MI, NJ, WN, WK, NST>;
+    using off_t = std::conditional_t<BIG, uint64_t, uint32_t>;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wn = w % WN, wk = w / WN;
+    const int lane = threadIdx.x & 63, fr = lane & 15, kg = lane >> 4;
+    const off_t K = A.k;
+    constexpr int WO = GU ? WN / 2 : WN;                   // waves side by side over the output columns
+    const bool up = GU && wn >= WO;
+    const int nw = n0 + 16 * NJ * (wn % WO);               // the wave's first column
+    constexpr int CPT = T == 16 ? 32 : 16;                 // 16-byte chunks of a tile per stage
+    // this k-group's stages t0 .. t1 - 1 of nk 32-row steps in all
+    const int nk = A.k / 32, ns = (nk + 1) / 2;
+    const int t0 = (int)((int64_t)ns * wk / WK), t1 = (int)((int64_t)ns * (wk + 1) / WK);
+    const int iters = (ns + WK - 1) / WK;
 
+    // Lane offsets of the wave's DMA instructions, rows, tiles and groups
+    // past the matrix clamped to its last; *back: what a lane of the second
+    // 32 rows steps back where the stage has only the first.
+    const int tlast = A.n / T - 1, tb = min(nw / T, tlast);
+    const char* cbase = reinterpret_cast<const char*>(up ? A.codes2 : A.codes) + (size_t)tb * A.k * (T / 2);
+    off_t co[NJ / 2];
+    uint32_t cback[NJ / 2];
+#pragma unroll
+    for (int q = 0; q < NJ / 2; ++q) {
+        const int tl = (64 * q + lane) / CPT, ch = ((64 * q + lane) % CPT) ^ (T == 16 ? tl & 3 : tl & 7);
+        co[q] = (off_t)(min(nw / T + tl, tlast) - tb) * K * (T / 2) + ch * 16;
+        cback[q] = ch >= CPT / 2 ? 32 * (T / 2) : 0;
+    }
+    const int glast = A.n / 32 - 1, gb = min(nw / 32, glast);
+    const char* sbase = reinterpret_cast<const char*>(up ? A.gscales2 : A.gscales) + (size_t)gb * A.k * 2;
+    const off_t so = ((off_t)(min(nw / 32 + (NJ == 4 ? lane / 32 : 0), glast) - gb) * K + 2 * (lane % 32)) * 2;
+    const uint32_t sback = lane % 32 >= 16 ? 64 : 0;
+    const char* xbase = reinterpret_cast<const char*>(A.x + (size_t)m0 * A.k);
+    constexpr int NX = (2 * MI + WN - 1) / WN;             // x instructions (8 rows each) of this wave
+    off_t xo[NX];
+    const uint32_t xch = (lane & 7) ^ (lane >> 3), xback = xch >= 4 ? 64 : 0;
+#pragma unroll
+    for (int q = 0; q < NX; ++q) {
+        const int r = 8 * min(wn * NX + q, 2 * MI - 1) + (lane >> 3);
+        xo[q] = (off_t)min(r, A.m - 1 - m0) * K * 2 + xch * 16;
+    }
+    constexpr int PER = NX + NJ / 2 + 1;                   // DMA instructions per wave and stage
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem + wk * NST * L::STAGE;
+    const char* sm = smem + wk * NST * L::STAGE;
+    auto dma = [](const char* base, off_t off, uint32_t lds) {
+        if constexpr (BIG) dma16(base + off, lds);
+        else dma16_off(base, off, lds);
+    };
+    auto issue = [&](int t, int buf) {
+        const bool half = 2 * t + 1 >= nk;                 // the last step of an odd count has no second one
+        const uint32_t lx = lds0 + buf * L::STAGE, lc = lx + L::X + wn * (L::C + L::S);
+#pragma unroll
+        for (int q = 0; q < NX; ++q)
+            dma(xbase + (size_t)t * 128, xo[q] - (half ? xback : 0), lx + 1024 * min(wn * NX + q, 2 * MI - 1));
+#pragma unroll
+        for (int q = 0; q < NJ / 2; ++q)
+            dma(cbase + (size_t)t * (64 * (T / 2)), co[q] - (half ? cback[q] : 0), lc + 1024 * q);
+        const off_t s = so - (half ? sback : 0);
+        if constexpr (BIG) dma4(sbase + (size_t)t * 128 + s, lc + L::C);
+        else dma4_off(sbase + (size_t)t * 128, s, lc + L::C);
+    };
+
+    const int mytile = (NJ * fr) / T;
+    const uint32_t sel = 0x0c040c00u + 0x00010001u * (((NJ * fr) % 8) / 2);   // byte of the lane's first column pair
     // the f16 exponent pattern 0x6400 (1024) of each half, held in a VGPR so
-    // that masking a nibble pair into it is one v_and_or_b32 (the mask is
-    // the instruction's one literal)
+    // that masking a nibble pair into it is one v_and_or_b32 (the mask is the
+    // instruction's one literal)
     uint32_t vmagic;
     asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(vmagic));
-    uint4 ra0, ra1;
-    uint32_t rb[4];
-    uint2 rs;                                            // RQ f16 scales of rows RQ rq .. +RQ-1
-#define GM_GLOAD(kt)                                                                   \
-    do {                                                                               \
-        const int k0_ = (kt) * GM_TK;                                                  \
-        ra0 = *reinterpret_cast<const uint4*>(xrow + k0_);                            \
-        if (XH == 16) ra1 = *reinterpret_cast<const uint4*>(xrow + k0_ + 8);          \
-        if (wthread) {                                                                 \
-            _Pragma("unroll") for (int i_ = 0; i_ < RQ; ++i_)                          \
-                rb[i_] = *reinterpret_cast<const uint32_t*>(bcodes + (size_t)(k0_ + i_) * cstride); \
-            if (RQ == 4) rs = *reinterpret_cast<const uint2*>(bsc + k0_);             \
-            else rs.x = *reinterpret_cast<const uint32_t*>(bsc + k0_);                \
-        }                                                                              \
-    } while (0)
-    // Columns 2b, 2b + 1 of a row pair come from byte b of each row's block.
-    // v_perm_b32 puts the first row's byte at bits 0-7 and the second's at
-    // bits 16-23 (of the words, and of the words shifted down by 4 for the
-    // high nibbles); masking a nibble pair into 0x6400 | q gives the f16 pair
-    // (1024 + q), and packed f16 ops make it s * (q - 8): exact, then one
-    // rounding of the product (the same bits as rounding s * (q - 8) from
-    // fp32).  Column n's four (two) rows are one 8-byte (4-byte) store.
-#define GM_BPAIR(v) (XBF16 ? f16x2_to_bf16x2(v) : __builtin_bit_cast(uint32_t, v))
-#define GM_LSTORE(buf)                                                                 \
-    do {                                                                               \
-        *reinterpret_cast<uint4*>(&sA[buf][ar][XH * ah]) = ra0;                        \
-        if (XH == 16) *reinterpret_cast<uint4*>(&sA[buf][ar][XH * ah + 8]) = ra1;      \
-        const half2 s01 = __builtin_bit_cast(half2, rs.x), s23 = __builtin_bit_cast(half2, rs.y); \
-        uint32_t rh[RQ];                                  /* high nibbles moved down once */ \
-        _Pragma("unroll") for (int i_ = 0; i_ < RQ; ++i_) rh[i_] = rb[i_] >> 4;       \
-        if (wthread) _Pragma("unroll") for (int b_ = 0; b_ < 4; ++b_) {                \
-            const uint32_t sel = 0x0c040c00u + 0x00010001u * b_;                       \
-            const half2 k1032 = half2{1032.0f16, 1032.0f16};                           \
-            const uint32_t p01 = __builtin_amdgcn_perm(rb[1], rb[0], sel);             \
-            const uint32_t q01 = __builtin_amdgcn_perm(rh[1], rh[0], sel);             \
-            const half2 l01 = (__builtin_bit_cast(half2, (p01 & 0x000f000fu) | vmagic) - k1032) * s01; \
-            const half2 h01 = (__builtin_bit_cast(half2, (q01 & 0x000f000fu) | vmagic) - k1032) * s01; \
-            if constexpr (RQ == 4) {                                                   \
-                const uint32_t p23 = __builtin_amdgcn_perm(rb[3], rb[2], sel);         \
-                const uint32_t q23 = __builtin_amdgcn_perm(rh[3], rh[2], sel);         \
-                const half2 l23 = (__builtin_bit_cast(half2, (p23 & 0x000f000fu) | vmagic) - k1032) * s23; \
-                const half2 h23 = (__builtin_bit_cast(half2, (q23 & 0x000f000fu) | vmagic) - k1032) * s23; \
-                *reinterpret_cast<uint2*>(&sB[buf][8 * c8 + 2 * b_][4 * rq]) = make_uint2(GM_BPAIR(l01), GM_BPAIR(l23)); \
-                *reinterpret_cast<uint2*>(&sB[buf][8 * c8 + 2 * b_ + 1][4 * rq]) = make_uint2(GM_BPAIR(h01), GM_BPAIR(h23)); \
-            } else {                                                                   \
-                *reinterpret_cast<uint32_t*>(&sB[buf][8 * c8 + 2 * b_][2 * rq]) = GM_BPAIR(l01); \
-                *reinterpret_cast<uint32_t*>(&sB[buf][8 * c8 + 2 * b_ + 1][2 * rq]) = GM_BPAIR(h01); \
-            }                                                                          \
-        }                                                                              \
-    } while (0)
 
+    // the MFMAs of rows 32 h .. +31 of a stage
+    auto step = [&](const char* sx, const char* sc, int h) {
+        uint32_t c[8];                                     // the lane's code word of rows 32 h + 8 kg .. +7
+        if constexpr (T == 16) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const uint32_t* p = reinterpret_cast<const uint32_t*>(
+                    sc + (mytile * CPT + 16 * h + 4 * kg + (r ^ (mytile & 3))) * 16) + ((NJ * fr) % 16) / 8;
+                c[2 * r] = p[0];
+                c[2 * r + 1] = p[2];
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                const uint4 v = *reinterpret_cast<const uint4*>(sc + (mytile * CPT + ((8 * h + 2 * kg + r) ^ (mytile & 7))) * 16);
+                c[4 * r] = v.x; c[4 * r + 1] = v.y; c[4 * r + 2] = v.z; c[4 * r + 3] = v.w;
+            }
+        }
+        const uint4 sv = *reinterpret_cast<const uint4*>(sc + L::C + (NJ * fr / 32) * 128 + 64 * h + 16 * kg);
+        const uint32_t s4[4] = {sv.x, sv.y, sv.z, sv.w};
+        // Columns 2 q, 2 q + 1 of the lane are the low and high nibbles of
+        // one byte of each row.  v_perm_b32 puts that byte of a row pair in
+        // the two halves; masked into 0x6400 they are 1024 + c and 1024 + 16
+        // c, and 1024 + c - 1032 and (1024 + 16 c) / 16 - 72 are c - 8
+        // exactly; times s is the one rounding (the same bits as rounding s *
+        // (c - 8) from fp32).
+        uint32_t b[NJ][4];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const half2 s2 = __builtin_bit_cast(half2, s4[p]);
+            auto put = [&](int j, half2 q8) {
+                const half2 v = q8 * s2;
+                b[j][p] = XBF16 ? f16x2_to_bf16x2(v) : __builtin_bit_cast(uint32_t, v);
+            };
+#pragma unroll
+            for (int q = 0; q < NJ / 2; ++q) {
+                const uint32_t wd = __builtin_amdgcn_perm(c[2 * p + 1], c[2 * p], sel + 0x00010001u * q);
+                put(2 * q, __builtin_bit_cast(half2, (wd & 0x000f000fu) | vmagic) - half2{1032.0f16, 1032.0f16});
+                put(2 * q + 1, __builtin_elementwise_fma(__builtin_bit_cast(half2, (wd & 0x00f000f0u) | vmagic),
+                                                         half2{0.0625f16, 0.0625f16}, half2{-72.0f16, -72.0f16}));
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+            const uint4 a = *reinterpret_cast<const uint4*>(sx + i * 2048 + fr * 128 + (((4 * h + kg) ^ (fr & 7)) << 4));
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const uint4 bj = make_uint4(b[j][0], b[j][1], b[j][2], b[j][3]);
+                if constexpr (XBF16)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        __builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, bj), acc[i][j], 0, 0, 0);
+                else
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                        __builtin_bit_cast(half8, a), __builtin_bit_cast(half8, bj), acc[i][j], 0, 0, 0);
+            }
+        }
+    };
+#pragma unroll
+    for (int p = 0; p < NST - 1; ++p)
+        if (t0 + p < t1) issue(t0 + p, p);
+    int buf = 0;
+    // Stage t has landed once at most the younger stage's DMAs are left; the
+    // barrier makes that true of every wave's part, and says that every wave
+    // has read stage t - 1 (lgkmcnt: its reads have returned), whose buffer
+    // is filled next.
+    static_assert(NST == 2 || NST == 3, "at most one younger stage in flight");
+    auto next = [&](int t) {
+        if (NST == 3 && t + 1 < t1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(PER) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (t + NST - 1 < t1) issue(t + NST - 1, buf == 0 ? NST - 1 : buf - 1);
+    };
+    // No branch around the MFMAs inside the loop: the accumulators would be
+    // copied at every merge.
+    const bool odd = t1 > t0 && 2 * t1 > nk;               // the range ends in a single step
+    const int tf = odd ? t1 - 1 : t1;
+    for (int t = t0; t < tf; ++t) {
+        next(t);
+        const char* sx = sm + buf * L::STAGE;
+        const char* sc = sx + L::X + wn * (L::C + L::S);
+        step(sx, sc, 0);
+        step(sx, sc, 1);
+        buf = buf == NST - 1 ? 0 : buf + 1;
+    }
+    if (odd) {
+        next(tf);
+        const char* sx = sm + buf * L::STAGE;
+        step(sx, sx + L::X + wn * (L::C + L::S), 0);
+    }
+    for (int it = t1 - t0; it < iters; ++it) asm volatile("s_barrier" ::: "memory");   // k-groups with fewer stages keep step
+}
+
+// GU: the gate/up form.  Waves 0 .. WN/2 - 1 of a k-group take the gate
+// weight's columns and the others the same columns of the up weight; the
+// epilogue writes silu(g) * u as bf16 (whose range, unlike f16's, holds any
+// product of the fp32 accumulators).
+template <bool XBF16, bool GU, int MI, int NJ, int WN, int WK, int NST, bool BIG = false>
+__device__ __forceinline__ void q4_gemm_body(const Q4GemmArgs& A) {
+    using L = Q4GemmLds<MI, NJ, WN, WK, NST>;
+    static_assert(!GU || WN % 2 == 0, "gate/up: half of the waves take the up weight");
+    static_assert(NJ == 2 || NJ == 4, "a lane's columns are one or two bytes of a row");
+    constexpr int WO = GU ? WN / 2 : WN, WAVES = WN * WK;
+    constexpr bool DIRECT = WK == 1 && !GU;                // one wave holds the whole sum of its outputs
+    constexpr int KB = WAVES * NJ;                         // KB of partials per 16 rows
+    constexpr int RB = L::BYTES > 65536 ? 64 : 32;         // KB of partials per round
+    constexpr int IR = KB * MI <= RB ? MI : (RB / KB > 1 ? RB / KB : 1);
+    constexpr int SMEM = DIRECT || L::BYTES > KB * IR * 1024 ? L::BYTES : KB * IR * 1024;
+    __shared__ __attribute__((aligned(1024))) char smem[SMEM];
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int wn = w % WN, wk = w / WN;
+    constexpr int NC = 16 * NJ * WO;
+    // consecutive workgroups walk n within one row block: its x rows are
+    // reused from L2 across its column tiles
+    const int nbn = (A.n + NC - 1) / NC;
+    const int bm = (int)(blockIdx.x / (uint32_t)nbn), bn = (int)(blockIdx.x % (uint32_t)nbn);
+    const int m0 = bm * 16 * MI, n0 = bn * NC;
     floatx4 acc[MI][NJ];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < NJ; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    auto mma = [](half8 a, half8 b, floatx4 c) {
-        if constexpr (XBF16)
-            return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b),
-                                                           c, 0, 0, 0);
-        else
-            return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-    };
+    if (A.tile == 16) q4_gemm_loop<XBF16, GU, MI, NJ, WN, WK, NST, 16, BIG>(A, m0, n0, smem, acc);
+    else q4_gemm_loop<XBF16, GU, MI, NJ, WN, WK, NST, 8, BIG>(A, m0, n0, smem, acc);
 
-    // Software pipeline over k steps, two LDS stages.  Entering iteration kt
-    // a wave holds step kt's fragments in registers, LDS stage (kt+1)&1 holds
-    // step kt+1 and the staging registers hold step kt+2's global data.
-    // Iteration kt runs step kt's MFMAs with step kt+1's fragment reads
-    // between them, stores step kt+2 into stage kt&1 (whose fragments every
-    // wave read before the previous barrier) and issues step kt+3's global
-    // loads; a barrier ends it.  The body is one basic block (the last
-    // iterations load a clamped step and store it into a stage nobody reads
-    // again), so the dequantization and the stores are scheduled between
-    // the MFMAs.  The k-step order of each accumulator is unchanged.
-    const int fr = lane & 15, fk = 8 * (lane >> 4);
-    GM_GLOAD(0);
-    GM_LSTORE(0);
-    GM_GLOAD(min(1, nk - 1));
-    GM_LSTORE(1);
-    GM_GLOAD(min(2, nk - 1));
-    __syncthreads();
-    half8 af[MI], bfr[NJ];
+    // n % 32 == 0 and col % NJ == 0: a lane's NJ columns are all in or all out
+    auto store = [&](int row, int col, float (&y)[NJ]) {
+        const size_t o = (size_t)row * A.n + col;
+        if (!GU && A.residual) {
 #pragma unroll
-    for (int i = 0; i < MI; ++i) af[i] = *reinterpret_cast<const half8*>(&sA[0][16 * MI * wm + 16 * i + fr][fk]);
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) bfr[j] = *reinterpret_cast<const half8*>(&sB[0][16 * NJ * wn + 16 * j + fr][fk]);
-    __syncthreads();
-    for (int kt = 0; kt < nk; ++kt) {
-        const int nb = (kt + 1) & 1;
-        half8 an[MI];
-#pragma unroll
-        for (int i = 0; i < MI; ++i) an[i] = *reinterpret_cast<const half8*>(&sA[nb][16 * MI * wm + 16 * i + fr][fk]);
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-#pragma unroll
-            for (int i = 0; i < MI; ++i) acc[i][j] = mma(af[i], bfr[j], acc[i][j]);
-            bfr[j] = *reinterpret_cast<const half8*>(&sB[nb][16 * NJ * wn + 16 * j + fr][fk]);
+            for (int j = 0; j < NJ; ++j) y[j] += A.residual[o + j];
         }
-        GM_LSTORE(kt & 1);
-        GM_GLOAD(min(kt + 3, nk - 1));
-        __builtin_amdgcn_iglp_opt(0);
+        if (GU || A.y_bf16) {
 #pragma unroll
-        for (int i = 0; i < MI; ++i) af[i] = an[i];
-        __syncthreads();
-    }
-#undef GM_GLOAD
-#undef GM_LSTORE
-#undef GM_BPAIR
-
-    // Epilogue through LDS.  A C fragment gives a lane 4 rows of one column
-    // (16 lanes: 32- or 64-byte pieces of a row), so each wave stages its
-    // tile 16 rows at a time in a private region of the idle W stages (the
-    // loop's last barrier ended every fragment read) and stores whole row
-    // segments, 16 bytes of fp32 per lane.  A wave reads back only what it
-    // wrote, and its LDS operations complete in order, so no barrier.  The
-    // row stride OC + 4 keeps the 64 lanes' stores in distinct banks.
-    constexpr int OC = GU ? 8 * NJ : 16 * NJ;              // output columns per wave
-    constexpr int EPS = OC + 4;
-    constexpr int LPR = OC / 4, RPI = 64 / LPR;            // lanes per staged row, rows per read
-    static_assert(WM * WN * 16 * EPS * 4 <= (int)sizeof(sB), "epilogue staging");
-    float* ep = reinterpret_cast<float*>(&sB[0][0][0]) + w * 16 * EPS;
-    const int oc0 = n0 + OC * wn;
+            for (int j = 0; j < NJ; j += 2)
+                *reinterpret_cast<uint32_t*>(A.y_bf16 + o + j) = pack_bf16x2(y[j], y[j + 1]);
+        } else {
 #pragma unroll
-    for (int i = 0; i < MI; ++i) {
+            for (int j = 0; j < NJ; ++j) A.y[o + j] = y[j];
+        }
+    };
+    if constexpr (DIRECT) {
+        const int col = n0 + 16 * NJ * wn + NJ * (lane & 15);
+        if (col >= A.n) return;
 #pragma unroll
-        for (int j = 0; j < NJ; j += (GU ? 2 : 1))
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                // gate/up: fragments j, j + 1 are the gate and up values of the same outputs
-                const float v = GU ? silu_fast(acc[i][j][e]) * acc[i][j + 1][e] : acc[i][j][e];
-                ep[(4 * (lane >> 4) + e) * EPS + (GU ? 8 : 16) * j + fr] = v;
-            }
+                const int row = m0 + 16 * i + 4 * (lane >> 4) + e;
+                float y[NJ];
 #pragma unroll
-        for (int r0 = 0; r0 < 16; r0 += RPI) {
-            const int r = r0 + lane / LPR, c = 4 * (lane % LPR);
-            const float4 v = *reinterpret_cast<const float4*>(&ep[r * EPS + c]);
-            const int row = m0 + 16 * MI * wm + 16 * i + r, col = oc0 + c;
-            if (row >= A.m || col >= A.n) continue;         // n % 32 == 0: the 4 columns are all in or all out
-            const size_t o = (size_t)row * A.n + col;
-            float4 y = v;
-            if (!GU && A.residual) {
-                const float4 rv = *reinterpret_cast<const float4*>(A.residual + o);
-                y = make_float4(v.x + rv.x, v.y + rv.y, v.z + rv.z, v.w + rv.w);
+                for (int j = 0; j < NJ; ++j) y[j] = acc[i][j][e];
+                if (row < A.m) store(row, col, y);
             }
-            if (GU || A.y_bf16)
-                *reinterpret_cast<uint2*>(A.y_bf16 + o) =
-                    make_uint2(pack_bf16x2(y.x, y.y), pack_bf16x2(y.z, y.w));
-            else
-                *reinterpret_cast<float4*>(A.y + o) = y;
+    } else {
+        // the k-groups' partial tiles meet where the stages were, IR row
+        // tiles a round, and are added in group order
+        float (*part)[WK][WN][4][64][NJ] = reinterpret_cast<float (*)[WK][WN][4][64][NJ]>(smem);
+#pragma unroll
+        for (int i0 = 0; i0 < MI; i0 += IR) {
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < IR; ++i)
+                if (i0 + i < MI)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j) part[i][wk][wn][e][lane][j] = acc[i0 + i][j][e];
+            __syncthreads();
+            for (int it = tid; it < IR * WO * 256; it += WAVES * 64) {
+                const int l = it & 63, e = (it >> 6) & 3, c = (it >> 8) % WO, i = (it >> 8) / WO;
+                const int row = m0 + 16 * (i0 + i) + 4 * (l >> 4) + e, col = n0 + 16 * NJ * c + NJ * (l & 15);
+                if (i0 + i >= MI || row >= A.m || col >= A.n) continue;
+                auto sum = [&](int v, float (&y)[NJ]) {
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j) y[j] = part[i][0][v][e][l][j];
+#pragma unroll
+                    for (int g = 1; g < WK; ++g)
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j) y[j] += part[i][g][v][e][l][j];
+                };
+                float y[NJ];
+                sum(c, y);
+                if constexpr (GU) {
+                    float u[NJ];
+                    sum(WO + c, u);
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j) y[j] = silu_fast(y[j]) * u[j];
+                }
+                store(row, col, y);
+            }
         }
     }
 }
 
-extern "C" __global__ __launch_bounds__(256, 2) void qm_q4_gemm(Q4GemmArgs A) { q4_gemm_body<false, false, 2, 2, 4, 8>(A); }
-extern "C" __global__ __launch_bounds__(256, 2) void qm_q4_gemm_xbf16(Q4GemmArgs A) { q4_gemm_body<true, false, 2, 2, 4, 8>(A); }
-extern "C" __global__ __launch_bounds__(256, 2) void qm_q4_gemm_gu(Q4GemmArgs A) { q4_gemm_body<false, true, 2, 2, 4, 8>(A); }
-extern "C" __global__ __launch_bounds__(256, 2) void qm_q4_gemm_gu_xbf16(Q4GemmArgs A) { q4_gemm_body<true, true, 2, 2, 4, 8>(A); }
-extern "C" __global__ __launch_bounds__(256, 2) void qm_q4_gemm_n128(Q4GemmArgs A) { q4_gemm_body<false, false, 2, 2, 4, 4>(A); }
-extern "C" __global__ __launch_bounds__(256, 2) void qm_q4_gemm_xbf16_n128(Q4GemmArgs A) { q4_gemm_body<true, false, 2, 2, 4, 4>(A); }
-extern "C" __global__ __launch_bounds__(256, 2) void qm_q4_gemm_m64(Q4GemmArgs A) { q4_gemm_body<false, false, 2, 2, 2, 4>(A); }
-extern "C" __global__ __launch_bounds__(256, 2) void qm_q4_gemm_xbf16_m64(Q4GemmArgs A) { q4_gemm_body<true, false, 2, 2, 2, 4>(A); }
-
-// n = 32 (the DeltaNet a/b projections, 8-column device tiles): 4096 x 2560
-// x 32 is too thin for LDS tiles, where each workgroup walks all k steps
-// behind one chain of loads.  Here a workgroup of four waves owns 16 rows
-// and deals the k steps to its waves round-robin.  Each wave builds its
-// MFMA operands straight from global memory: the x row piece (lane: row
-// lane & 15, k 8 (lane >> 4) .. +7) is the A operand as loaded; for the B
-// operand of column c the lane loads rows k .. k+7 of c's tile (32
-// contiguous bytes), takes nibble c & 7 of each and forms the f16 pairs
-// s * (q - 8) with the same magic-number arithmetic as the staged form (for
-// bf16 x, rounded on to bf16).  No LDS until the end, where the four
-// partial sums meet and are added in a fixed order.
-template <bool XBF16>
-__device__ __forceinline__ void q4_gemm_n32_body(const Q4GemmArgs& A) {
-    __shared__ floatx4 part[4][2][64];                   // [wave][column tile][lane]
-    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-    const int m0 = (int)blockIdx.x * 16, K = A.k, nk = K / GM_TK;
-    const int fr = lane & 15, kg = lane >> 4;
-    const uint16_t* xr = A.x + (size_t)min(m0 + fr, A.m - 1) * K + 8 * kg;
-    const int sh = 4 * (fr & 7);                         // nibble of column 16 j + fr in its row word
-    const uint8_t* cb[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) cb[j] = A.codes + (size_t)(2 * j + (fr >> 3)) * K * 4 + 32 * kg;
-    const uint16_t* sb = A.gscales + 8 * kg;             // one 32-column group: scales [k]
-    uint32_t vmagic;
-    asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(vmagic));
-    floatx4 acc[2] = {floatx4{0.0f, 0.0f, 0.0f, 0.0f}, floatx4{0.0f, 0.0f, 0.0f, 0.0f}};
-#pragma unroll 4
-    for (int kt = w; kt < nk; kt += 4) {
-        const int k0 = kt * GM_TK;
-        const half8 a = __builtin_bit_cast(half8, *reinterpret_cast<const uint4*>(xr + k0));
-        const uint4 sc = *reinterpret_cast<const uint4*>(sb + k0);
-        const uint32_t s4[4] = {sc.x, sc.y, sc.z, sc.w};
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const uint4 c0 = *reinterpret_cast<const uint4*>(cb[j] + (size_t)k0 * 4);
-            const uint4 c1 = *reinterpret_cast<const uint4*>(cb[j] + (size_t)k0 * 4 + 16);
-            const uint32_t wd[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-            uint32_t bw[4];
-#pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                const uint32_t q0 = (wd[2 * p] >> sh) & 0xfu, q1 = (wd[2 * p + 1] >> sh) & 0xfu;
-                const half2 v = (__builtin_bit_cast(half2, (q0 | (q1 << 16)) | vmagic) - half2{1032.0f16, 1032.0f16}) *
-                                __builtin_bit_cast(half2, s4[p]);
-                bw[p] = XBF16 ? f16x2_to_bf16x2(v) : __builtin_bit_cast(uint32_t, v);
-            }
-            const half8 bv = __builtin_bit_cast(half8, make_uint4(bw[0], bw[1], bw[2], bw[3]));
-            if constexpr (XBF16)
-                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, bv),
-                                                                 acc[j], 0, 0, 0);
-            else
-                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bv, acc[j], 0, 0, 0);
-        }
+#define Q4_GEMM(NAME, XB, GU, MI, NJ, WN, WK, NST, OCC, ...)                                       \
+    extern "C" __global__ __launch_bounds__(64 * WN * WK, OCC) void NAME(Q4GemmArgs A) {          \
+        q4_gemm_body<XB, GU, MI, NJ, WN, WK, NST, ##__VA_ARGS__>(A);                               \
     }
-#pragma unroll
-    for (int j = 0; j < 2; ++j) part[w][j][lane] = acc[j];
-    __syncthreads();
-    if (w != 0) return;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const floatx4 y = ((part[0][j][lane] + part[1][j][lane]) + part[2][j][lane]) + part[3][j][lane];
-        const int col = 16 * j + fr;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int row = m0 + 4 * kg + e;
-            if (row >= A.m) continue;
-            const size_t o = (size_t)row * A.n + col;
-            float v = y[e];
-            if (A.residual) v += A.residual[o];
-            if (A.y_bf16) A.y_bf16[o] = f32_to_bf16(v);
-            else A.y[o] = v;
-        }
-    }
-}
-extern "C" __global__ __launch_bounds__(256) void qm_q4_gemm_n32(Q4GemmArgs A) { q4_gemm_n32_body<false>(A); }
-extern "C" __global__ __launch_bounds__(256) void qm_q4_gemm_xbf16_n32(Q4GemmArgs A) { q4_gemm_n32_body<true>(A); }
+#define Q4_GEMM_PLAIN(MI, NJ, WN, WK, NST, OCC, ...)                                               \
+    Q4_GEMM(qm_q4_gemm_f16_m##MI##n##NJ##w##WN##k##WK, false, false, MI, NJ, WN, WK, NST, OCC)     \
+    Q4_GEMM(qm_q4_gemm_bf16_m##MI##n##NJ##w##WN##k##WK, true, false, MI, NJ, WN, WK, NST, OCC)
+#define Q4_GEMM_GATE_UP(MI, NJ, WN, WK, NST, OCC, ...)                                             \
+    Q4_GEMM(qm_q4_gemm_gu_f16_m##MI##n##NJ##w##WN##k##WK, false, true, MI, NJ, WN, WK, NST, OCC)   \
+    Q4_GEMM(qm_q4_gemm_gu_bf16_m##MI##n##NJ##w##WN##k##WK, true, true, MI, NJ, WN, WK, NST, OCC)
+QM_Q4_TILES_PAIRED(Q4_GEMM_PLAIN)
+QM_Q4_TILES_SINGLE(Q4_GEMM_PLAIN)
+QM_Q4_TILES_PAIRED(Q4_GEMM_GATE_UP)
+Q4_GEMM(qm_q4_gemm_f16_big, false, false, 1, 2, 2, 4, 3, 4, true)
+Q4_GEMM(qm_q4_gemm_bf16_big, true, false, 1, 2, 2, 4, 3, 4, true)
+Q4_GEMM(qm_q4_gemm_gu_f16_big, false, true, 1, 2, 2, 4, 3, 4, true)
+Q4_GEMM(qm_q4_gemm_gu_bf16_big, true, true, 1, 2, 2, 4, 3, 4, true)
 
 // rms_norm (1 + gamma, eps 1e-6; gemv.rs:571-579) of each of m rows of f32
 // x [m][k], written as the f16 input of qm_q4_gemm; without a norm weight,

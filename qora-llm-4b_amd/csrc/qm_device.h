@@ -128,4 +128,18 @@ QM_DEV void dma16(const void* gsrc, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
                  :: "v"(gsrc), "s"(lds) : "memory", "m0");
 }
+// The same from a wave-uniform base and a 32-bit lane offset, and both forms
+// with 4 bytes per lane (lane l writes lds + 4 l).
+QM_DEV void dma16_off(const void* base, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :: "v"(off), "s"(base), "s"(lds) : "memory", "m0");
+}
+QM_DEV void dma4(const void* gsrc, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
+                 :: "v"(gsrc), "s"(lds) : "memory", "m0");
+}
+QM_DEV void dma4_off(const void* base, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
+                 :: "v"(off), "s"(base), "s"(lds) : "memory", "m0");
+}
 #pragma clang diagnostic pop

@@ -12,6 +12,7 @@
 #include "qm_kernel_args.h"
 #include "qm_gqa_plan.h"
 #include "qm_noalloc.h"
+#include "qm_q4_tiles.h"
 
 #include <hip/hip_runtime_api.h>
 #include <dlfcn.h>
@@ -51,10 +52,8 @@ struct qm_context {
     hipFunction_t f_q4_gemv_inter = nullptr;   // 4096 < k <= 9216 (the MLP's intermediate size)
     hipFunction_t f_q4_repack = nullptr;
     hipFunction_t f_q4_gate_up = nullptr;
-    hipFunction_t f_q4_gemm[2][2] = {};  // [x bf16][gate/up form]
-    hipFunction_t f_q4_gemm_n128[2] = {}; // [x bf16]: 128 x 128 tiles for narrow outputs
-    hipFunction_t f_q4_gemm_m64[2] = {};  // [x bf16]: 64 x 128 tiles
-    hipFunction_t f_q4_gemm_n32[2] = {};  // [x bf16]: n = 32, 16 rows per 4-wave workgroup, k split over the waves
+    hipFunction_t f_q4_gemm[2][2][qm_q4::kNumTiles] = {};  // [x bf16][gate/up form][tile]
+    hipFunction_t f_q4_gemm_big[2][2] = {};                // 64-bit lane offsets
     hipFunction_t f_rms_f16 = nullptr;
     hipFunction_t f_lm_head = nullptr;
     hipFunction_t f_embed = nullptr;
@@ -363,16 +362,14 @@ int32_t qm_create(qm_context** out, const qm_config* cfg, const char* code_objec
     if (st == QM_OK) st = load_function(c, mods[5], "qm_q4_gemv_inter", &c->f_q4_gemv_inter);
     if (st == QM_OK) st = load_function(c, mods[5], "qm_q4_repack", &c->f_q4_repack);
     if (st == QM_OK) st = load_function(c, mods[5], "qm_q4_gate_up", &c->f_q4_gate_up);
-    if (st == QM_OK) st = load_function(c, mods[5], "qm_q4_gemm", &c->f_q4_gemm[0][0]);
-    if (st == QM_OK) st = load_function(c, mods[5], "qm_q4_gemm_xbf16", &c->f_q4_gemm[1][0]);
-    if (st == QM_OK) st = load_function(c, mods[5], "qm_q4_gemm_gu", &c->f_q4_gemm[0][1]);
-    if (st == QM_OK) st = load_function(c, mods[5], "qm_q4_gemm_gu_xbf16", &c->f_q4_gemm[1][1]);
-    if (st == QM_OK) st = load_function(c, mods[5], "qm_q4_gemm_n128", &c->f_q4_gemm_n128[0]);
-    if (st == QM_OK) st = load_function(c, mods[5], "qm_q4_gemm_xbf16_n128", &c->f_q4_gemm_n128[1]);
-    if (st == QM_OK) st = load_function(c, mods[5], "qm_q4_gemm_m64", &c->f_q4_gemm_m64[0]);
-    if (st == QM_OK) st = load_function(c, mods[5], "qm_q4_gemm_xbf16_m64", &c->f_q4_gemm_m64[1]);
-    if (st == QM_OK) st = load_function(c, mods[5], "qm_q4_gemm_n32", &c->f_q4_gemm_n32[0]);
-    if (st == QM_OK) st = load_function(c, mods[5], "qm_q4_gemm_xbf16_n32", &c->f_q4_gemm_n32[1]);
+    for (int i = 0; i < 4; ++i) {
+        const int xb = i & 1, gu = i >> 1;
+        const std::string stem = std::string("qm_q4_gemm_") + (gu ? "gu_" : "") + (xb ? "bf16_" : "f16_");
+        for (int t = 0; t < qm_q4::kNumTiles && st == QM_OK; ++t)
+            if (!gu || qm_q4::kTiles[t].wn % 2 == 0)
+                st = load_function(c, mods[5], (stem + qm_q4::kTiles[t].name).c_str(), &c->f_q4_gemm[xb][gu][t]);
+        if (st == QM_OK) st = load_function(c, mods[5], (stem + "big").c_str(), &c->f_q4_gemm_big[xb][gu]);
+    }
     if (st == QM_OK) st = load_function(c, mods[5], "qm_rms_norm_f16", &c->f_rms_f16);
     if (st == QM_OK) st = load_function(c, mods[6], "qm_q4_lm_head", &c->f_lm_head);
     if (st == QM_OK) st = load_function(c, mods[6], "qm_q4_embed", &c->f_embed);
@@ -1112,6 +1109,20 @@ int32_t q4_gemm_check(qm_context* c, const char* name, int32_t m, int32_t k, int
         return fail(c, QM_ERR_INVALID_ARG, "%s: x_dtype %d (QM_F16 or QM_BF16)", name, x_dtype);
     return QM_OK;
 }
+
+int32_t q4_gemm_launch(qm_context* c, qm_stream stream, const Q4GemmArgs& ga, int32_t x_dtype, bool gate_up,
+                       const char* what) {
+    const int xb = x_dtype == QM_BF16;
+    int ti = qm_q4::pick_tile(ga.m, ga.k, ga.n, xb, gate_up, c->num_cu);
+    hipFunction_t f = c->f_q4_gemm[xb][gate_up][ti];
+    if (ga.k > QM_Q4_GEMM_MAX_K32) {
+        ti = qm_q4::kBigTile;
+        f = c->f_q4_gemm_big[xb][gate_up];
+    }
+    const qm_q4::Tile& t = qm_q4::kTiles[ti];
+    return launch(c, f, static_cast<uint32_t>(qm_q4::tile_grid(t, ga.m, ga.n, gate_up)),
+                  static_cast<uint32_t>(64 * t.wn * t.wk), ga, pick(c, stream), what);
+}
 }  // namespace
 
 int32_t qm_q4_gemm(qm_context* c, qm_stream stream, int32_t m, int32_t k, int32_t n, const uint16_t* x,
@@ -1125,22 +1136,7 @@ int32_t qm_q4_gemm(qm_context* c, qm_stream stream, int32_t m, int32_t k, int32_
     if (!all_aligned16({x, codes, gscales, residual, y, y_bf16}))
         return fail(c, QM_ERR_INVALID_ARG, "qm_q4_gemm: device pointers must be 16-byte aligned");
     Q4GemmArgs ga{x, codes, gscales, nullptr, nullptr, y, y_bf16, residual, m, k, n, QM_Q4_TILE(n)};
-    const int xb = x_dtype == QM_BF16;
-    auto tiles = [&](int64_t tm, int64_t tn) { return (m + tm - 1) / tm * ((n + tn - 1) / tn); };
-    const int64_t two_per_cu = 2 * static_cast<int64_t>(c->num_cu);
-    // the widest tile that still gives two workgroups per CU; n = 32 (the
-    // DeltaNet a/b projections) a k-split kernel of 16 rows per workgroup
-    if (n <= 32)
-        return launch(c, c->f_q4_gemm_n32[xb], static_cast<uint32_t>((m + 15) / 16), 256, ga, pick(c, stream),
-                      "qm_q4_gemm");
-    if (tiles(128, 256) >= two_per_cu)
-        return launch(c, c->f_q4_gemm[xb][0], static_cast<uint32_t>(tiles(128, 256)), 256, ga, pick(c, stream),
-                      "qm_q4_gemm");
-    if (tiles(128, 128) >= two_per_cu)
-        return launch(c, c->f_q4_gemm_n128[xb], static_cast<uint32_t>(tiles(128, 128)), 256, ga, pick(c, stream),
-                      "qm_q4_gemm");
-    return launch(c, c->f_q4_gemm_m64[xb], static_cast<uint32_t>(tiles(64, 128)), 256, ga, pick(c, stream),
-                  "qm_q4_gemm");
+    return q4_gemm_launch(c, stream, ga, x_dtype, false, "qm_q4_gemm");
 }
 
 int32_t qm_q4_gemm_gate_up(qm_context* c, qm_stream stream, int32_t m, int32_t k, int32_t n, const uint16_t* x,
@@ -1155,8 +1151,7 @@ int32_t qm_q4_gemm_gate_up(qm_context* c, qm_stream stream, int32_t m, int32_t k
         return fail(c, QM_ERR_INVALID_ARG, "qm_q4_gemm_gate_up: device pointers must be 16-byte aligned");
     Q4GemmArgs ga{x, gate_codes, gate_gscales, up_codes, up_gscales, nullptr, out_bf16, nullptr, m, k, n,
                   QM_Q4_TILE(n)};
-    const uint32_t grid = static_cast<uint32_t>((m + 127) / 128) * static_cast<uint32_t>((n + 127) / 128);
-    return launch(c, c->f_q4_gemm[x_dtype == QM_BF16][1], grid, 256, ga, pick(c, stream), "qm_q4_gemm_gate_up");
+    return q4_gemm_launch(c, stream, ga, x_dtype, true, "qm_q4_gemm_gate_up");
 }
 
 }  // extern "C"

@@ -244,10 +244,8 @@ def test_rms_norm_f16(ctx):
     assert np.array_equal(ctx.download(out, (m, k), np.uint16), W.f16_bits(x))
 
 
-# Tile shapes on 256 CUs: m = 1930 on the 8192-wide weight (512 tiles of
-# 128 x 256) and m = 3300 on the 2560-wide one (520 tiles of 128 x 128)
-# take the wide kernels, the smaller cases 64 x 128 tiles, and n = 32 the
-# one-wave 16 x 32 kernel.
+# Projection shapes from one row to thousands, so that calls take small and
+# large workgroup tiles.
 @pytest.mark.parametrize("name,m,mode", [("in_proj_qkv", 200, "bf16"), ("in_proj_z", 37, "bf16"),
                                          ("out_proj", 64, "residual"), ("in_proj_a", 130, "f32"),
                                          ("down_proj", 129, "residual"), ("k_proj", 1, "f32"),
@@ -437,6 +435,83 @@ def test_q4_gemm_bf16_rows_past_f16_range_match_unscaled_rows(ctx):
     assert np.array_equal(got[m:], got[:m] * np.float32(2.0 ** 20))
     ref = O.q4_gemm(base, packed, scales).astype(np.float64)
     assert np.all(np.abs(got[:m] - ref) <= BF16_W_EPS * _mag(base, packed, scales) + 1e-30)
+
+
+# Sizes at which a call on 256 CUs takes each workgroup tile (qm_q4_tiles.h),
+# ragged in every direction: rows and columns that end inside a tile, n in
+# both device layouts (8-column tiles below 4096), k of an odd number of
+# 32-row steps and k with fewer 64-row stages than k-groups.
+GEMM_TILES = [("m1n2w1k16", 1, 2592, 2592), ("m1n2w1k16", 1, 544, 5152), ("m1n2w1k8", 16, 32, 96),
+              ("m1n2w1k8", 1, 96, 4128), ("m1n2w2k4", 33, 96, 4128), ("m2n2w1k8", 17, 2592, 4128),
+              ("m2n2w1k8", 49, 544, 2592), ("m3n2w1k8", 45, 2592, 4128), ("m3n2w1k8", 97, 2592, 2592),
+              ("m3n2w2k4", 65, 96, 4128), ("m4n2w1k8", 49, 544, 5152), ("m4n2w1k8", 161, 2592, 2592),
+              ("m4n2w2k4", 161, 544, 4128), ("m4n2w2k4", 300, 544, 2592), ("m4n2w4k2", 161, 96, 4128),
+              ("m4n4w2k4", 385, 1056, 4128), ("m4n4w2k4", 641, 1056, 2592), ("m6n4w2k4", 385, 544, 5152),
+              ("m6n4w4k1", 500, 32, 4128), ("m6n4w4k2", 900, 96, 5152), ("m8n4w4k1", 1537, 96, 8192),
+              ("m8n4w4k2", 1300, 96, 5152), ("gate/up m1n2w2k4", 1, 2592, 2592), ("gate/up m3n2w2k4", 17, 2592, 4128),
+              ("gate/up m4n2w2k4", 161, 544, 2592), ("gate/up m4n2w4k2", 65, 96, 4128),
+              ("gate/up m4n4w2k4", 161, 1056, 4128), ("gate/up m4n4w2k4", 900, 2592, 1056),
+              ("gate/up m6n4w2k4", 193, 544, 5152), ("gate/up m6n4w4k1", 193, 32, 4128),
+              ("gate/up m6n4w4k2", 257, 96, 8192), ("gate/up m8n4w4k1", 900, 96, 8192),
+              ("gate/up m8n4w4k2", 641, 96, 5152)]
+
+
+@pytest.mark.parametrize("x_dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("tile,m,k,n", GEMM_TILES)
+def test_q4_gemm_tiles(ctx, tile, m, k, n, x_dtype):
+    """Each tile against the stated arithmetic in float64: x times W as the
+    MFMA multiplies it (f16(s (q - 8)), for a bf16 x on to bf16).  What is
+    left is the fp32 accumulation, at most (k + 8) 2^-24 of sum |x w| in any
+    order; gate/up carries both sums' through silu(g) u (|silu'| <= 1.1) and
+    rounds to bf16."""
+    rng = np.random.default_rng(m * 31 + k + n)
+    pairs = [W.q4_random_weight(k, n, rng) for _ in range(2 if tile.startswith("gate/up") else 1)]
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    bits = W.bf16_bits(x) if x_dtype == "bf16" else W.f16_bits(x)
+    xv = (W.bf16_value(bits) if x_dtype == "bf16" else W.f16_value(bits)).astype(np.float64)
+    ws = [(_w_bf16(*p) if x_dtype == "bf16" else W.f16_value(W.f16_bits(W.q4_dequant(*p)))).astype(np.float64)
+          for p in pairs]
+    sums, mags = [xv @ w for w in ws], [(k + 8) * 2.0 ** -24 * (np.abs(xv) @ np.abs(w)) for w in ws]
+    dev = [repack(ctx, *p) for p in pairs]
+    dt = M.QM_BF16 if x_dtype == "bf16" else M.QM_F16
+    print(f"case: q4 gemm tile {tile} m={m} k={k} n={n} {x_dtype}", flush=True)
+    if len(pairs) == 1:
+        y = ctx.upload(np.full((m, n), np.nan, np.float32))
+        ctx.q4_gemm(m, k, n, ctx.upload(bits), *dev[0], y=y, x_dtype=dt)
+        got = ctx.download(y, (m, n), np.float32).astype(np.float64)
+        ref, bound = sums[0], mags[0]
+    else:
+        y = ctx.upload(np.full((m, n), 0x7fc0, np.uint16))
+        ctx.q4_gemm_gate_up(m, k, n, ctx.upload(bits), *dev[0], *dev[1], y, x_dtype=dt)
+        got = W.bf16_value(ctx.download(y, (m, n), np.uint16)).astype(np.float64)
+        silu = sums[0] / (1.0 + np.exp(-sums[0]))
+        ref = silu * sums[1]
+        bound = 1.1 * mags[0] * np.abs(sums[1]) + np.abs(silu) * mags[1] + (2.0 ** -8 + 1e-6) * np.abs(ref)
+    err = np.abs(got - ref) / (bound + 1e-30)
+    print(f"max|d|/bound {err.max():.3e}")
+    assert np.all(err <= 1.0)
+
+
+def test_q4_gemm_long_k(ctx):
+    """k past the tiles' 32-bit lane offsets takes the form with 64-bit ones.
+    Rounding errors of 8.4 million fp32 additions: 1e-4 of sum |x w| is far
+    above their random walk and far below a dropped or repeated part of k."""
+    m, k, n = 2, (1 << 23) + 32, 32
+    rng = np.random.default_rng(23)
+    packed, scales = W.q4_random_weight(k, n, rng)
+    x16 = W.f16_bits(rng.standard_normal((m, k), dtype=np.float32))
+    codes, gsc = repack(ctx, packed, scales)
+    y = ctx.alloc(m * n * 4)
+    print("case: q4 gemm long k", flush=True)
+    ctx.q4_gemm(m, k, n, ctx.upload(x16), codes, gsc, y=y)
+    got = ctx.download(y, (m, n), np.float32).astype(np.float64)
+    ref, mag = np.zeros((m, n)), np.zeros((m, n))
+    for i in range(0, k, 1 << 20):
+        w = W.q4_dequant(packed[i:i + (1 << 20)], scales[i:i + (1 << 20)]).astype(np.float64)
+        xv = W.f16_value(x16[:, i:i + (1 << 20)]).astype(np.float64)
+        ref += xv @ w
+        mag += np.abs(xv) @ np.abs(w)
+    assert np.all(np.abs(got - ref) <= 1e-4 * mag)
 
 
 def test_q4_gemm_errors(ctx):
