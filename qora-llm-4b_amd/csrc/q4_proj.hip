@@ -432,7 +432,8 @@ extern "C" __global__ __launch_bounds__(256) void qm_q4_repack(Q4RepackArgs A) {
 // one lane at a time: measured 60 cache accesses per load instruction, the L1
 // at one access per cycle the whole launch).  16-byte chunks are xor-swizzled
 // in each row or tile so that the operand reads meet no bank conflict
-// (SQ_LDS_BANK_CONFLICT 0).  One barrier per stage.
+// (SQ_LDS_BANK_CONFLICT 0).  One barrier per stage where the waves of a
+// k-group share its x rows (WN > 1), none where a k-group is one wave.
 //
 // What bounds it.  Large m: issue slots.  Per step of 32 rows a 128 x 64 wave
 // tile issues 32 MFMAs and ~80 VALU instructions (1.75 per weight pair and
@@ -449,14 +450,14 @@ extern "C" __global__ __launch_bounds__(256) void qm_q4_repack(Q4RepackArgs A) {
 // workgroup into LDS, 128 x 256 tiles, one barrier per 32 rows), us, same
 // box, rotating weights:
 //   m x k x n            before    now
-//   45 x 2560 x 8192       39.1    8.1     (DeltaNet in_proj_qkv)
-//   45 x 9216 x 2560      141.9   14.4     (down_proj, bf16 x)
-//   300 x 9216 x 2560     141     36
+//   48 x 2560 x 8192       39.4    6.9     (DeltaNet in_proj_qkv)
+//   48 x 9216 x 2560      141.9   13.3     (down_proj, bf16 x)
+//   300 x 9216 x 2560     140     33
 //   700 x 4096 x 2560      64     28       (o_proj, bf16 x)
-//   4096 x 2560 x 8192    187    152       (1.13 PFLOP/s)
-//   4096 x 9216 x 2560    271    238
-//   4096 x 2560 x 32        9.9    5.6     (in_proj_a / b)
-//   4096 x 2560 x 9216 gate/up  406    337  (1.15 PFLOP/s)
+//   4096 x 2560 x 8192    187    151       (1.14 PFLOP/s)
+//   4096 x 9216 x 2560    271    235
+//   4096 x 2560 x 32        9.9    5.1     (in_proj_a / b)
+//   4096 x 2560 x 9216 gate/up  406    331  (1.17 PFLOP/s)
 // Tried and no faster: dequantizing the next step's operand between the
 // MFMAs of this one (explicit interleave; 0-3% either way), two LDS stages
 // instead of three (0-2%), and reading x and codes without LDS (3-4 x slower
@@ -493,14 +494,15 @@ __device__ __forceinline__ void q4_gemm_loop(const Q4GemmArgs& A, int m0, int n0
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wn = w % WN, wk = w / WN;
     const int lane = threadIdx.x & 63, fr = lane & 15, kg = lane >> 4;
     const off_t K = A.k;
-    constexpr int WO = GU ? WN / 2 : WN;                   // waves side by side over the output columns
-    const bool up = GU && wn >= WO;
+    constexpr int WO = GU && WN > 1 ? WN / 2 : WN;         // waves side by side over the output columns
+    constexpr int KG = GU && WN == 1 ? WK / 2 : WK;        // k-groups per weight
+    const bool up = GU && (WN > 1 ? wn >= WO : wk >= KG);
     const int nw = n0 + 16 * NJ * (wn % WO);               // the wave's first column
     constexpr int CPT = T == 16 ? 32 : 16;                 // 16-byte chunks of a tile per stage
     // this k-group's stages t0 .. t1 - 1 of nk 32-row steps in all
     const int nk = A.k / 32, ns = (nk + 1) / 2;
-    const int t0 = (int)((int64_t)ns * wk / WK), t1 = (int)((int64_t)ns * (wk + 1) / WK);
-    const int iters = (ns + WK - 1) / WK;
+    const int g = wk % KG, t0 = (int)((int64_t)ns * g / KG), t1 = (int)((int64_t)ns * (g + 1) / KG);
+    const int iters = (ns + KG - 1) / KG;
 
     // Lane offsets of the wave's DMA instructions, rows, tiles and groups
     // past the matrix clamped to its last; *back: what a lane of the second
@@ -621,11 +623,14 @@ __device__ __forceinline__ void q4_gemm_loop(const Q4GemmArgs& A, int m0, int n0
     // Stage t has landed once at most the younger stage's DMAs are left; the
     // barrier makes that true of every wave's part, and says that every wave
     // has read stage t - 1 (lgkmcnt: its reads have returned), whose buffer
-    // is filled next.
+    // is filled next.  A k-group of one wave (WN = 1) fills and reads its own
+    // buffers only: its waits are enough, and its waves drift apart, one's
+    // dequantization beside another's MFMAs.
     static_assert(NST == 2 || NST == 3, "at most one younger stage in flight");
     auto next = [&](int t) {
-        if (NST == 3 && t + 1 < t1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(PER) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (NST == 3 && t + 1 < t1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(PER) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        if (WN > 1) asm volatile("s_barrier" ::: "memory");
         if (t + NST - 1 < t1) issue(t + NST - 1, buf == 0 ? NST - 1 : buf - 1);
     };
     // No branch around the MFMAs inside the loop: the accumulators would be
@@ -645,19 +650,22 @@ __device__ __forceinline__ void q4_gemm_loop(const Q4GemmArgs& A, int m0, int n0
         const char* sx = sm + buf * L::STAGE;
         step(sx, sx + L::X + wn * (L::C + L::S), 0);
     }
-    for (int it = t1 - t0; it < iters; ++it) asm volatile("s_barrier" ::: "memory");   // k-groups with fewer stages keep step
+    // k-groups with fewer stages keep step
+    for (int it = t1 - t0; WN > 1 && it < iters; ++it) asm volatile("s_barrier" ::: "memory");
 }
 
 // GU: the gate/up form.  Waves 0 .. WN/2 - 1 of a k-group take the gate
-// weight's columns and the others the same columns of the up weight; the
-// epilogue writes silu(g) * u as bf16 (whose range, unlike f16's, holds any
-// product of the fp32 accumulators).
+// weight's columns and the others the same columns of the up weight (WN = 1:
+// the first half of the k-groups the gate weight, the second half the up
+// weight); the epilogue writes silu(g) * u as bf16 (whose range, unlike
+// f16's, holds any product of the fp32 accumulators).
 template <bool XBF16, bool GU, int MI, int NJ, int WN, int WK, int NST, bool BIG = false>
 __device__ __forceinline__ void q4_gemm_body(const Q4GemmArgs& A) {
     using L = Q4GemmLds<MI, NJ, WN, WK, NST>;
-    static_assert(!GU || WN % 2 == 0, "gate/up: half of the waves take the up weight");
+    static_assert(!GU || (WN == 1 ? WK : WN) % 2 == 0, "gate/up: half of the waves take the up weight");
     static_assert(NJ == 2 || NJ == 4, "a lane's columns are one or two bytes of a row");
-    constexpr int WO = GU ? WN / 2 : WN, WAVES = WN * WK;
+    constexpr int WO = GU && WN > 1 ? WN / 2 : WN, WAVES = WN * WK;
+    constexpr int KG = GU && WN == 1 ? WK / 2 : WK;        // k-groups per weight
     constexpr bool DIRECT = WK == 1 && !GU;                // one wave holds the whole sum of its outputs
     constexpr int KB = WAVES * NJ;                         // KB of partials per 16 rows
     constexpr int RB = L::BYTES > 65536 ? 64 : 32;         // KB of partials per round
@@ -728,19 +736,20 @@ __device__ __forceinline__ void q4_gemm_body(const Q4GemmArgs& A) {
                 const int l = it & 63, e = (it >> 6) & 3, c = (it >> 8) % WO, i = (it >> 8) / WO;
                 const int row = m0 + 16 * (i0 + i) + 4 * (l >> 4) + e, col = n0 + 16 * NJ * c + NJ * (l & 15);
                 if (i0 + i >= MI || row >= A.m || col >= A.n) continue;
-                auto sum = [&](int v, float (&y)[NJ]) {
+                auto sum = [&](int g0, int v, float (&y)[NJ]) {
 #pragma unroll
-                    for (int j = 0; j < NJ; ++j) y[j] = part[i][0][v][e][l][j];
+                    for (int j = 0; j < NJ; ++j) y[j] = part[i][g0][v][e][l][j];
 #pragma unroll
-                    for (int g = 1; g < WK; ++g)
+                    for (int g = 1; g < KG; ++g)
 #pragma unroll
-                        for (int j = 0; j < NJ; ++j) y[j] += part[i][g][v][e][l][j];
+                        for (int j = 0; j < NJ; ++j) y[j] += part[i][g0 + g][v][e][l][j];
                 };
                 float y[NJ];
-                sum(c, y);
+                sum(0, c, y);
                 if constexpr (GU) {
                     float u[NJ];
-                    sum(WO + c, u);
+                    if constexpr (WN == 1) sum(KG, c, u);
+                    else sum(0, WO + c, u);
 #pragma unroll
                     for (int j = 0; j < NJ; ++j) y[j] = silu_fast(y[j]) * u[j];
                 }
@@ -760,13 +769,15 @@ __device__ __forceinline__ void q4_gemm_body(const Q4GemmArgs& A) {
 #define Q4_GEMM_GATE_UP(MI, NJ, WN, WK, NST, OCC, ...)                                             \
     Q4_GEMM(qm_q4_gemm_gu_f16_m##MI##n##NJ##w##WN##k##WK, false, true, MI, NJ, WN, WK, NST, OCC)   \
     Q4_GEMM(qm_q4_gemm_gu_bf16_m##MI##n##NJ##w##WN##k##WK, true, true, MI, NJ, WN, WK, NST, OCC)
+QM_Q4_TILES_ONE_WAVE(Q4_GEMM_PLAIN)
 QM_Q4_TILES_PAIRED(Q4_GEMM_PLAIN)
-QM_Q4_TILES_SINGLE(Q4_GEMM_PLAIN)
+QM_Q4_TILES_ODD(Q4_GEMM_PLAIN)
+QM_Q4_TILES_ONE_WAVE(Q4_GEMM_GATE_UP)
 QM_Q4_TILES_PAIRED(Q4_GEMM_GATE_UP)
-Q4_GEMM(qm_q4_gemm_f16_big, false, false, 1, 2, 2, 4, 3, 4, true)
-Q4_GEMM(qm_q4_gemm_bf16_big, true, false, 1, 2, 2, 4, 3, 4, true)
-Q4_GEMM(qm_q4_gemm_gu_f16_big, false, true, 1, 2, 2, 4, 3, 4, true)
-Q4_GEMM(qm_q4_gemm_gu_bf16_big, true, true, 1, 2, 2, 4, 3, 4, true)
+Q4_GEMM(qm_q4_gemm_f16_big, false, false, 1, 2, 1, 8, 3, 4, true)
+Q4_GEMM(qm_q4_gemm_bf16_big, true, false, 1, 2, 1, 8, 3, 4, true)
+Q4_GEMM(qm_q4_gemm_gu_f16_big, false, true, 1, 2, 1, 8, 3, 4, true)
+Q4_GEMM(qm_q4_gemm_gu_bf16_big, true, true, 1, 2, 1, 8, 3, 4, true)
 
 // rms_norm (1 + gamma, eps 1e-6; gemv.rs:571-579) of each of m rows of f32
 // x [m][k], written as the f16 input of qm_q4_gemm; without a norm weight,

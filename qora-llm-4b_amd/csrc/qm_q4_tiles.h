@@ -10,32 +10,39 @@
 // CU, and per workgroup where a CU has several, for an f16 and a bf16 x (the
 // bf16 form converts W once more).
 //
+// Gate/up needs two equal halves of a workgroup, one per weight: of the WN
+// waves side by side, or of the k-groups where WN is 1.
+//
 // X(MI, NJ, WN, WK, NST, OCC, alone f16, shared f16, alone bf16, shared bf16)
 #pragma once
 #include <stdint.h>
 
-// tiles with an even WN: the gate/up form takes these (half of the waves hold
-// the gate weight's columns, half the up weight's)
-#define QM_Q4_TILES_PAIRED(X)                             \
-    X(1, 2, 2, 4, 3, 4, 446, 438, 643, 545)               \
-    X(3, 2, 2, 4, 2, 4, 637, 618, 808, 668)               \
-    X(4, 2, 2, 4, 3, 2, 779, 959, 942, 996)               \
-    X(4, 2, 4, 2, 3, 4, 718, 651, 850, 713)               \
-    X(4, 4, 2, 4, 3, 2, 1242, 1506, 1462, 1552)           \
-    X(6, 4, 2, 4, 2, 2, 1658, 1936, 1824, 1949)           \
-    X(6, 4, 4, 1, 3, 2, 904, 732, 1038, 819)              \
-    X(6, 4, 4, 2, 3, 2, 1432, 1643, 1686, 1743)           \
-    X(8, 4, 4, 1, 3, 2, 1098, 912, 1230, 954)             \
-    X(8, 4, 4, 2, 3, 2, 1737, 2042, 1967, 2084)
-#define QM_Q4_TILES_SINGLE(X)                             \
-    X(1, 2, 1, 16, 3, 4, 878, 1456, 1185, 1456)           \
-    X(1, 2, 1, 8, 3, 4, 440, 512, 647, 580)               \
-    X(2, 2, 1, 8, 3, 2, 618, 962, 789, 899)               \
-    X(3, 2, 1, 8, 2, 2, 780, 1197, 959, 1066)             \
-    X(4, 2, 1, 8, 2, 2, 952, 1425, 1132, 1248)
+#define QM_Q4_TILES_ONE_WAVE(X)                 \
+    X(1, 2, 1, 8, 3, 4, 424, 445, 595, 546)     \
+    X(1, 2, 1, 16, 2, 4, 733, 1161, 1061, 1320) \
+    X(1, 4, 1, 8, 2, 4, 608, 690, 994, 921)     \
+    X(2, 2, 1, 8, 2, 2, 488, 731, 680, 787)     \
+    X(2, 4, 1, 8, 2, 2, 787, 1092, 1100, 1207)  \
+    X(3, 2, 1, 8, 2, 2, 623, 903, 773, 890)     \
+    X(3, 4, 1, 8, 2, 2, 1058, 1370, 1285, 1426) \
+    X(4, 2, 1, 8, 2, 2, 792, 1105, 896, 1031)   \
+    X(5, 4, 1, 4, 2, 1, 932, 1050, 1008, 1068)  \
+    X(6, 4, 1, 4, 2, 1, 1075, 1210, 1097, 1170) \
+    X(8, 4, 1, 4, 2, 1, 1348, 1463, 1364, 1442)
+#define QM_Q4_TILES_PAIRED(X)                   \
+    X(3, 2, 2, 4, 2, 4, 641, 627, 797, 669)     \
+    X(4, 2, 4, 2, 3, 4, 696, 649, 864, 715)     \
+    X(6, 4, 2, 4, 2, 2, 1650, 1967, 1797, 1931) \
+    X(6, 4, 4, 1, 3, 2, 888, 734, 1006, 812)    \
+    X(6, 4, 4, 2, 3, 2, 1427, 1652, 1681, 1760) \
+    X(8, 4, 4, 1, 3, 2, 1089, 907, 1220, 942)   \
+    X(8, 4, 4, 2, 3, 2, 1736, 2032, 1992, 2105)
+// an odd number of k-groups: no gate/up form
+#define QM_Q4_TILES_ODD(X)                      \
+    X(4, 4, 1, 7, 2, 2, 1220, 1597, 1378, 1508)
 
 // Above this k the tiles' 32-bit lane offsets do not reach (128 rows of x);
-// the (1, 2, 2, 4) tile has a form with 64-bit addresses.
+// the first tile has a form with 64-bit ones.
 #define QM_Q4_GEMM_MAX_K32 (1 << 23)
 
 #ifndef __HIP_DEVICE_COMPILE__
@@ -49,13 +56,16 @@ struct Tile {
 
 #define QM_Q4_TILE_ROW(MI, NJ, WN, WK, NST, OCC, AF, SF, AB, SB) \
     {"m" #MI "n" #NJ "w" #WN "k" #WK, MI, NJ, WN, WK, {AF, AB}, {SF, SB}},
-constexpr Tile kTiles[] = {QM_Q4_TILES_PAIRED(QM_Q4_TILE_ROW) QM_Q4_TILES_SINGLE(QM_Q4_TILE_ROW)};
+constexpr Tile kTiles[] = {QM_Q4_TILES_ONE_WAVE(QM_Q4_TILE_ROW) QM_Q4_TILES_PAIRED(QM_Q4_TILE_ROW)
+                           QM_Q4_TILES_ODD(QM_Q4_TILE_ROW)};
 #undef QM_Q4_TILE_ROW
 constexpr int kBigTile = 0;      // the tile of the form with 64-bit lane offsets
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 
+inline bool has_gate_up(const Tile& t) { return (t.wn == 1 ? t.wk : t.wn) % 2 == 0; }
+
 inline int64_t tile_grid(const Tile& t, int64_t m, int64_t n, bool gate_up) {
-    const int64_t rows = 16 * t.mi, cols = 16 * t.nj * (gate_up ? t.wn / 2 : t.wn);
+    const int64_t rows = 16 * t.mi, cols = 16 * t.nj * (gate_up && t.wn > 1 ? t.wn / 2 : t.wn);
     return (m + rows - 1) / rows * ((n + cols - 1) / cols);
 }
 
@@ -65,14 +75,15 @@ inline int64_t tile_grid(const Tile& t, int64_t m, int64_t n, bool gate_up) {
 // loads less per product, a small one, or one that splits k over its waves,
 // fills the CUs and shortens the chain of stages when there are few rows.
 // Over the measured sizes the choice was within 1% of the best of these tiles
-// on average (15% at worst).
+// on average (20% at worst).
 inline int pick_tile(int64_t m, int64_t k, int64_t n, bool bf16, bool gate_up, int num_cu) {
     int best = -1;
     int64_t best_ns = 0;
     for (int i = 0; i < kNumTiles; ++i) {
         const Tile& t = kTiles[i];
-        if (gate_up && t.wn % 2) continue;
-        const int64_t stages = ((k / 32 + 1) / 2 + t.wk - 1) / t.wk;
+        if (gate_up && !has_gate_up(t)) continue;
+        const int64_t groups = gate_up && t.wn == 1 ? t.wk / 2 : t.wk;
+        const int64_t stages = ((k / 32 + 1) / 2 + groups - 1) / groups;
         const int64_t per_cu = (tile_grid(t, m, n, gate_up) + num_cu - 1) / num_cu;
         const int64_t shared = per_cu * t.shared[bf16];
         const int64_t ns = stages * (per_cu == 1 || shared < t.alone[bf16] ? t.alone[bf16] : shared);

@@ -441,19 +441,30 @@ def test_q4_gemm_bf16_rows_past_f16_range_match_unscaled_rows(ctx):
 # ragged in every direction: rows and columns that end inside a tile, n in
 # both device layouts (8-column tiles below 4096), k of an odd number of
 # 32-row steps and k with fewer 64-row stages than k-groups.
-GEMM_TILES = [("m1n2w1k16", 1, 2592, 2592), ("m1n2w1k16", 1, 544, 5152), ("m1n2w1k8", 16, 32, 96),
-              ("m1n2w1k8", 1, 96, 4128), ("m1n2w2k4", 33, 96, 4128), ("m2n2w1k8", 17, 2592, 4128),
-              ("m2n2w1k8", 49, 544, 2592), ("m3n2w1k8", 45, 2592, 4128), ("m3n2w1k8", 97, 2592, 2592),
-              ("m3n2w2k4", 65, 96, 4128), ("m4n2w1k8", 49, 544, 5152), ("m4n2w1k8", 161, 2592, 2592),
-              ("m4n2w2k4", 161, 544, 4128), ("m4n2w2k4", 300, 544, 2592), ("m4n2w4k2", 161, 96, 4128),
-              ("m4n4w2k4", 385, 1056, 4128), ("m4n4w2k4", 641, 1056, 2592), ("m6n4w2k4", 385, 544, 5152),
-              ("m6n4w4k1", 500, 32, 4128), ("m6n4w4k2", 900, 96, 5152), ("m8n4w4k1", 1537, 96, 8192),
-              ("m8n4w4k2", 1300, 96, 5152), ("gate/up m1n2w2k4", 1, 2592, 2592), ("gate/up m3n2w2k4", 17, 2592, 4128),
-              ("gate/up m4n2w2k4", 161, 544, 2592), ("gate/up m4n2w4k2", 65, 96, 4128),
-              ("gate/up m4n4w2k4", 161, 1056, 4128), ("gate/up m4n4w2k4", 900, 2592, 1056),
-              ("gate/up m6n4w2k4", 193, 544, 5152), ("gate/up m6n4w4k1", 193, 32, 4128),
-              ("gate/up m6n4w4k2", 257, 96, 8192), ("gate/up m8n4w4k1", 900, 96, 8192),
-              ("gate/up m8n4w4k2", 641, 96, 5152)]
+GEMM_TILES = [("m1n2w1k16", 1, 544, 4128), ("m1n2w1k16", 1, 544, 32), ("m1n2w1k8", 1, 352, 4128),
+              ("m1n2w1k8", 1, 352, 32), ("m2n2w1k8", 17, 352, 4128), ("m2n2w1k8", 49, 352, 2592),
+              ("m2n4w1k8", 65, 352, 4128), ("m3n2w1k8", 33, 352, 8192), ("m3n2w1k8", 97, 352, 2592),
+              ("m3n2w2k4", 97, 544, 4128), ("m3n2w2k4", 193, 544, 2592), ("m3n4w1k8", 97, 352, 4128),
+              ("m3n4w1k8", 193, 352, 2592), ("m4n2w1k8", 900, 352, 544), ("m4n2w4k2", 161, 32, 4128),
+              ("m4n2w4k2", 300, 32, 2592), ("m4n4w1k7", 161, 352, 4128), ("m4n4w1k7", 300, 352, 2592),
+              ("m5n4w1k4", 193, 352, 4128), ("m5n4w1k4", 385, 352, 2592), ("m6n4w1k4", 257, 544, 4128),
+              ("m6n4w1k4", 500, 544, 2592), ("m6n4w2k4", 385, 352, 5152), ("m6n4w2k4", 900, 352, 2592),
+              ("m6n4w4k1", 385, 32, 5152), ("m6n4w4k1", 900, 32, 2592), ("m6n4w4k2", 1000, 96, 4128),
+              ("m6n4w4k2", 1537, 96, 2592), ("m8n4w1k4 (bf16 x)", 193, 544, 8192), ("m8n4w4k1", 1537, 32, 4128), ("m8n4w4k2", 1537, 96, 4128),
+              ("gate/up m1n2w1k16", 1, 352, 4128), ("gate/up m1n2w1k16", 1, 352, 32),
+              ("gate/up m1n2w1k8", 1, 544, 4128), ("gate/up m1n2w1k8", 1, 544, 32),
+              ("gate/up m2n2w1k8", 17, 352, 4128), ("gate/up m2n2w1k8", 49, 352, 2592),
+              ("gate/up m2n4w1k8", 65, 352, 4128), ("gate/up m3n2w1k8", 33, 352, 8192),
+              ("gate/up m3n2w1k8", 97, 352, 2592), ("gate/up m3n4w1k8", 97, 544, 4128),
+              ("gate/up m3n4w1k8", 193, 544, 2592), ("gate/up m4n2w1k8", 900, 352, 544),
+              ("gate/up m4n2w4k2", 161, 352, 4128), ("gate/up m4n2w4k2", 300, 352, 2592),
+              ("gate/up m5n4w1k4", 193, 352, 4128), ("gate/up m5n4w1k4", 385, 352, 2592),
+              ("gate/up m6n4w1k4", 257, 352, 4128), ("gate/up m6n4w1k4", 500, 352, 2592),
+              ("gate/up m6n4w2k4", 257, 544, 4128), ("gate/up m6n4w2k4", 500, 544, 2592),
+              ("gate/up m6n4w4k1", 193, 32, 4128), ("gate/up m6n4w4k1", 385, 32, 2592),
+              ("gate/up m6n4w4k2", 385, 96, 5152), ("gate/up m6n4w4k2", 900, 96, 2592),
+              ("gate/up m8n4w4k1", 700, 32, 4128), ("gate/up m8n4w4k1", 1300, 32, 2592),
+              ("gate/up m8n4w4k2", 700, 96, 4128), ("gate/up m8n4w4k2", 1300, 96, 2592)]
 
 
 @pytest.mark.parametrize("x_dtype", ["f16", "bf16"])
