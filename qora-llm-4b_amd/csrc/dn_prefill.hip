@@ -128,19 +128,20 @@ QM_DEV void chunk_prep(const DnPrefillArgs& A, const int (&chb)[NP], _Float16 (*
                 x[r][2 * e + 1] = bf16_to_f32((uint16_t)(wv[e] >> 16));
             }
         }
-        // the masks are wave-uniform branches: interior chunks skip them
-        if (c == 0) {                              // x_{-3..-1} from the conv buffer
+        // the masks are wave-uniform branches: interior chunks skip them, and
+        // only wave 0 (tokens 0 .. 15) reaches back before the sequence
+        if (c == 0 && __builtin_amdgcn_readfirstlane(tid >> 6) == 0) {   // x_{-3..-1} from the conv buffer
             asm volatile("" ::: "memory");        // keep these loads inside the branch
+            float cb[24];                         // the 8 channels' buffers, oldest first: 96 contiguous bytes
 #pragma unroll
-            for (int r = 0; r < 3; ++r) {
-                const int t = 4 * tg - 3 + r;
-                const int tb = min(t, -1);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float cbv = A.conv_buf[(size_t)(ch0 + e) * 3 + 3 + tb];
-                    x[r][e] = t < 0 ? cbv : x[r][e];
-                }
+            for (int q = 0; q < 6; ++q) {
+                const float4 v = ld4(A.conv_buf + (size_t)ch0 * 3 + 4 * q);
+                cb[4 * q] = v.x; cb[4 * q + 1] = v.y; cb[4 * q + 2] = v.z; cb[4 * q + 3] = v.w;
             }
+#pragma unroll
+            for (int r = 0; r < 3; ++r)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[r][e] = tg == 0 ? cb[3 * e + r] : x[r][e];
             // the selects complete here, inside the branch: no load of it
             // is then pending where the paths join, and other chunks'
             // arithmetic waits only for the rows it uses
@@ -225,7 +226,9 @@ QM_DEV void chunk_vmax(float (&vm)[8], float (*red)[QM_DN_HD], float& om) {
 // gates are formed first, the second head's v once the first head is done
 // with the per-head LDS.  At ~79 KB of LDS two workgroups share a CU, so
 // one's stalls (loads, barriers, MFMA and LDS latency) can be filled by the
-// other's work; an 8-wave workgroup doing both heads at once (119 KB, one per
+// other's work; in a short sequence (args.split), where that would leave CUs
+// idle, a workgroup takes one v-head, preparing q and k a second time beside
+// the other head's workgroup instead of one head after the other.  An 8-wave workgroup doing both heads at once (119 KB, one per
 // CU) measured 74.5 us against 71 us for a 4096-token layer.
 // [W | U~] = (I + A)^-1 [diag(beta gamma) K | diag(beta) V] is solved by block
 // forward substitution over the four 16-token blocks b:
@@ -247,7 +250,9 @@ void qm_dn_prefill_chunk(DnPrefillArgs A) {
 
     const int tid = threadIdx.x;
     // GVA: v-heads 2 qkh and 2 qkh + 1 read qk-head qkh (gemv.rs:1160)
-    const int c = blockIdx.x / QM_DN_QK_HEADS, qkh = blockIdx.x % QM_DN_QK_HEADS;
+    const int per_chunk = A.split ? QM_DN_V_HEADS : QM_DN_QK_HEADS;
+    const int c = blockIdx.x / per_chunk, hb = blockIdx.x % per_chunk, qkh = A.split ? hb >> 1 : hb;
+    const int hh0 = A.split ? hb & 1 : 0, hh1 = A.split ? hh0 + 1 : 2;   // its v-heads 2 qkh + hh
     const int t0 = c * CHK;
     const bool tail = t0 + CHK > A.T;              // last chunk, partly past the sequence
     _Float16 (&Vs)[CHK][136] = H.Vs;
@@ -265,14 +270,14 @@ void qm_dn_prefill_chunk(DnPrefillArgs A) {
         const int cg = tid & 15;
         const int chb[2] = {qkh * QM_DN_HD + 8 * cg, QM_DN_QK_DIM + qkh * QM_DN_HD + 8 * cg};
         _Float16 (*const dst[2])[136] = {Qs, Ks};
-        const int chv[1] = {2 * QM_DN_QK_DIM + (2 * qkh) * QM_DN_HD + 8 * cg};
+        const int chv[1] = {2 * QM_DN_QK_DIM + (2 * qkh + hh0) * QM_DN_HD + 8 * cg};
         _Float16 (*const dsv[1])[136] = {Vs};
         float ga = 0.0f, gb = 0.0f, vm[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) vm[e] = 0.0f;
         chunk_prep<2, 2>(A, chb, dst, qkh, t0, c, tail, true, ga, gb, vm);
         chunk_prep<1, 0>(A, chv, dsv, qkh, t0, c, tail, false, ga, gb, vm);
-        chunk_vmax(vm, vred[0], om_v0);
+        chunk_vmax(vm, vred[hh0], om_v0);
         if (tid < 2 * CHK) {
             // log alpha = -exp(A_log) softplus(a + dt_bias), beta = sigmoid(b);
             // padded tokens get alpha = 1, beta = 0 (no effect on the state);
@@ -308,7 +313,7 @@ void qm_dn_prefill_chunk(DnPrefillArgs A) {
     }
 
 #pragma unroll 1
-    for (int hh = 0; hh < 2; ++hh) {
+    for (int hh = hh0; hh < hh1; ++hh) {
         // The thread's indices, re-derived from an opaque copy in each pass:
         // otherwise the compiler computes every lane-dependent address and
         // constant of the body once, ahead of the loop, and keeps them all
@@ -322,8 +327,8 @@ void qm_dn_prefill_chunk(DnPrefillArgs A) {
         const ChunkGates& G = gts[hh];
         // largest magnitude this thread converts to an f16 operand in the
         // solve (q, k, A, P and K~ are bounded by the normalisation)
-        float om = hh == 0 ? om_v0 : 0.0f;
-        if (hh == 1) {
+        float om = hh == hh0 ? om_v0 : 0.0f;
+        if (hh != hh0) {
             // the second head's v, into the per-head LDS the first head has
             // finished with (the barrier after its statistics)
             const int cg = tid & 15;
@@ -333,7 +338,7 @@ void qm_dn_prefill_chunk(DnPrefillArgs A) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) vm[e] = 0.0f;
             chunk_prep<1, 0>(A, chb, dst, qkh, t0, c, tail, false, ga, gb, vm);
-            chunk_vmax(vm, vred[1], om);
+            chunk_vmax(vm, vred[hh], om);
             __syncthreads();
         }
 

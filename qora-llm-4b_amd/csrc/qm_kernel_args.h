@@ -113,6 +113,7 @@ struct DnPrefillArgs {
     int32_t* mode;
     int32_t T;
     int32_t nc;
+    int32_t split;           // chunk kernel: one workgroup per (chunk, v-head) instead of per (chunk, qk-head)
 };
 
 // GQA causal prefill.  kvf is a workspace copy of the f16 K and V, per kv

@@ -116,6 +116,22 @@ def test_prefill_long_warm(ctx, T):
     assert np.array_equal(cb, rcb)
 
 
+@pytest.mark.parametrize("T", [2, 3, 1024, 1025])
+def test_prefill_workgroup_forms(ctx, T):
+    """The chunk kernel's edges on 256 CUs: 16 chunks are the last to take a
+    workgroup per v-head, 17 the first to take one per qk-head; sequences
+    shorter than the conv history keep part of the entering one."""
+    w = W.dn_prefill_workload(T, seed=11 + T)
+    r = np.random.default_rng(T)
+    w["state0"] = (0.02 * r.standard_normal((32, 128, 128))).astype(np.float32)
+    w["conv_buf0"] = r.standard_normal((8192, 3)).astype(np.float32)
+    print(f"case: dn prefill workgroup forms T={T}", flush=True)
+    o, S, cb = run_prefill(ctx, w, T)
+    ro, rS, rcb = run_oracle(w, T)
+    assert rel(o, ro) <= RTOL and rel(S, rS) <= RTOL
+    assert np.array_equal(cb, rcb)
+
+
 # v channels 5, 900, 2100, 4000 lie in v-heads 0, 7, 16 and 31
 OUTLIER_V = [4096 + 5, 4096 + 900, 4096 + 2100, 4096 + 4000]
 OUTLIER_HEADS = [0, 7, 16, 31]
