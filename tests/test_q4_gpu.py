@@ -244,6 +244,23 @@ def test_rms_norm_f16(ctx):
     assert np.array_equal(ctx.download(out, (m, k), np.uint16), W.f16_bits(x))
 
 
+@pytest.mark.parametrize("k", [4, 1020, 1028, 4096, 4100])
+def test_rms_norm_f16_row_lengths(ctx, k):
+    """Rows around the edges of the in-register form (1024 values per load, at
+    most 4096) and the first that is read twice: one f16 rounding, plus the
+    fp32 sum of squares in another order."""
+    rng = np.random.default_rng(k)
+    m = 3
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    gamma = W.f16_bits(0.1 * rng.standard_normal(k))
+    out = ctx.alloc(m * k * 2)
+    print(f"case: rms norm k={k}", flush=True)
+    ctx.rms_norm_f16(m, k, ctx.upload(x), ctx.upload(gamma), out)
+    got = W.f16_value(ctx.download(out, (m, k), np.uint16)).astype(np.float64)
+    ref = np.stack([O.rms_norm(r, gamma) for r in x]).astype(np.float64)
+    assert np.all(np.abs(got - ref) <= np.abs(ref) * 2.0 ** -10 + 1e-7)
+
+
 # Projection shapes from one row to thousands, so that calls take small and
 # large workgroup tiles.
 @pytest.mark.parametrize("name,m,mode", [("in_proj_qkv", 200, "bf16"), ("in_proj_z", 37, "bf16"),
