@@ -61,6 +61,8 @@ struct qm_context {
     hipFunction_t f_sample_pen = nullptr;
     hipFunction_t f_sample = nullptr;
     hipFunction_t f_sample_select = nullptr;
+    hipFunction_t f_sample_slices = nullptr;
+    hipFunction_t f_sample_draw = nullptr;
     int lm_head_hidden = 0;              // the hidden size lm_head_wg_per_cu was computed for
     int lm_head_wg_per_cu = 1;
     int dnp_chunk_threads = 0;     // the DeltaNet prefill chunk kernel's workgroup size (its launch bounds)
@@ -378,6 +380,8 @@ int32_t qm_create(qm_context** out, const qm_config* cfg, const char* code_objec
     if (st == QM_OK) st = load_function(c, mods[7], "qm_sample_penalties", &c->f_sample_pen);
     if (st == QM_OK) st = load_function(c, mods[7], "qm_sample_top_k", &c->f_sample);
     if (st == QM_OK) st = load_function(c, mods[7], "qm_sample_select", &c->f_sample_select);
+    if (st == QM_OK) st = load_function(c, mods[7], "qm_sample_slices", &c->f_sample_slices);
+    if (st == QM_OK) st = load_function(c, mods[7], "qm_sample_draw", &c->f_sample_draw);
     if (st == QM_OK &&
         (hipFuncGetAttribute(&c->q4_threads, HIP_FUNC_ATTRIBUTE_MAX_THREADS_PER_BLOCK, c->f_q4_gemv) != hipSuccess ||
          hipFuncGetAttribute(&c->q4_gu_threads, HIP_FUNC_ATTRIBUTE_MAX_THREADS_PER_BLOCK, c->f_q4_gate_up) !=
@@ -1088,9 +1092,26 @@ int32_t qm_sample(qm_context* c, qm_stream stream, int32_t vocab, float* logits,
     hipStream_t s = pick(c, stream);
     int32_t st = ensure(c, s, kSampleWsBytes);
     if (st != QM_OK) return st;
+    const int64_t k = greedy ? 1 : std::min(p->top_k, vocab);
+    // The short way needs k slices (the k-th largest slice maximum bounds the
+    // candidates) and a wave that holds the probabilities: k <= 64, slices of
+    // 1024, 512 or 256 logits, at most 256 of them (vocab <= 262144).
+    if (k <= 64) {
+        int32_t slice = 1024;
+        while (slice > 256 && (vocab + slice - 1) / slice < k) slice /= 2;
+        const int32_t ns = (vocab + slice - 1) / slice;
+        if (ns >= k) {
+            SampleArgs sa{logits,     generated,     rng_state,      token_out,  top_ids,
+                          top_probs,  vocab,         n_generated,    p->top_k,   p->banned_id,
+                          p->flags,   p->temperature, p->top_p,      p->repetition_penalty, p->presence_penalty,
+                          static_cast<uint64_t*>(c->ws), slice, 0};
+            st = launch(c, c->f_sample_slices, static_cast<uint32_t>(ns), 256, sa, s, "qm_sample_slices");
+            if (st != QM_OK) return st;
+            return launch(c, c->f_sample_draw, 1, 1024, sa, s, "qm_sample_draw");
+        }
+    }
     // stage 1 slices: 1024 m logits each, so that slices x k candidates fit
     // the stage-2 sort (8192)
-    const int64_t k = greedy ? 1 : std::min(p->top_k, vocab);
     int64_t m = 1;
     while ((vocab + 1024 * m - 1) / (1024 * m) * k > 8192) ++m;
     const int64_t chunk = 1024 * m, nw = (vocab + chunk - 1) / chunk;

@@ -26,6 +26,20 @@
 //      reference calls libm expf, correctly rounded but for rare half-way
 //      cases).
 // Greedy (temperature <= 0) is the same selection with k = 1.
+//
+// For k up to 64 and enough slices (the host's rule) a shorter way, two launches:
+//   qm_sample_slices: each workgroup applies the penalties to its slice of the
+//      vocabulary and writes the slice's largest key;
+//   qm_sample_draw (one workgroup): the k-th largest of those keys is a lower
+//      bound of the k-th largest logit, and only slices that reach it hold
+//      candidates, so some 20 slices are read instead of sorting each; the
+//      candidates are ranked by counting, and one wave draws, its lanes
+//      holding the probabilities.
+// What bounded the longer way was its chain of steps, not bytes: penalties 4.8
+// us, select 11.8 (four radix passes, a scan and a sort per slice), merge and
+// draw 14.6 (20 rounds of a 64-lane maximum, then one thread's loads from
+// LDS); now 5.3 and 11.2 us (248,320 logits, top 20, presence penalty over 1000
+// ids).
 #include "qm_device.h"
 #include "qm_kernel_args.h"
 
@@ -34,6 +48,8 @@
 #define SMP_MAX_CAND 8192          // stage-1 candidates (slices x k), merged in LDS
 #define SMP_MAX_LISTS 256          // stage-1 slices (vocabulary / 1024 at most)
 #define SMP_MAX_VOCAB 262144       // the presence bitmap in LDS (32 KB)
+#define SMP_MAX_SLICE 1024         // logits per workgroup of qm_sample_slices (256, 512 or 1024)
+#define SMP_DRAW_CAND 4096         // candidates qm_sample_draw ranks by counting
 
 // Larger logit -> larger key; -0 == +0; NaN below every number.
 QM_DEV uint32_t logit_key(float v) {
@@ -78,6 +94,61 @@ extern "C" __global__ __launch_bounds__(SMP_THREADS) void qm_sample_penalties(Sa
     }
     __syncthreads();
     if (tid == 0 && A.banned >= 0 && A.banned < A.vocab) A.logits[A.banned] = -__builtin_inff();
+}
+
+// The penalties and the largest key of one slice [w CH, (w + 1) CH) of the
+// vocabulary, in place: the same arithmetic per logit as
+// qm_sample_penalties (a logit's penalties depend on no other's).
+extern "C" __global__ __launch_bounds__(256) void qm_sample_slices(SampleArgs A) {
+#pragma clang fp contract(off)
+    __shared__ uint32_t seen[SMP_MAX_SLICE / 32];
+    __shared__ uint32_t wmax[4];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int s0 = blockIdx.x * A.chunk, s1 = min(s0 + A.chunk, A.vocab);
+    const int n = A.n_generated;
+    const bool repeat = A.repetition_penalty > 1.0f && n > 0, presence = A.presence_penalty > 0.0f && n > 0;
+    if (presence && tid < SMP_MAX_SLICE / 32) seen[tid] = 0u;
+    // generate.rs:58-69: lane i holds the i-th id of the window; the first
+    // occurrence of an id applies its penalty as often as the id occurs
+    if (repeat && tid < 64) {
+        const int window = min(n, 64);
+        const int tok = lane < window ? A.generated[n - window + lane] : -1;
+        int count = 0, first = 64;
+        for (int i = 63; i >= 0; --i) {
+            const bool same = __builtin_amdgcn_readlane(tok, i) == tok;
+            count += same;
+            first = same ? i : first;
+        }
+        if (tok >= s0 && tok < s1 && first == lane) {
+            float l = A.logits[tok];
+            for (int i = 0; i < count; ++i)
+                l = l > 0.0f ? __fdiv_rn(l, A.repetition_penalty) : __fmul_rn(l, A.repetition_penalty);
+            A.logits[tok] = l;
+        }
+    }
+    __syncthreads();
+    // generate.rs:72-82: once per distinct id
+    if (presence)
+        for (int i = tid; i < n; i += 256) {
+            const int tok = A.generated[i];
+            if (tok < s0 || tok >= s1) continue;
+            const uint32_t bit = 1u << ((tok - s0) & 31);
+            if (!(atomicOr(&seen[(tok - s0) >> 5], bit) & bit)) A.logits[tok] = __fsub_rn(A.logits[tok], A.presence_penalty);
+        }
+    __syncthreads();
+    if (tid == 0 && A.banned >= s0 && A.banned < s1) A.logits[A.banned] = -__builtin_inff();
+    __syncthreads();
+    uint32_t m = 0;
+#pragma unroll
+    for (int j = 0; j < SMP_MAX_SLICE / 256; ++j) {
+        const int i = s0 + tid + 256 * j;
+        if (i < s1) m = max(m, logit_key(A.logits[i]));
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off));
+    if (lane == 0) wmax[tid >> 6] = m;
+    __syncthreads();
+    if (tid == 0) reinterpret_cast<uint32_t*>(A.cand)[blockIdx.x] = max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
 }
 
 // Candidate order: key descending, then index ascending (descending for
@@ -348,4 +419,173 @@ extern "C" __global__ __launch_bounds__(SMP_THREADS) void qm_sample_top_k(Sample
         }
     }
     A.token_out[0] = tok;
+}
+
+// The composites (key, index) of the logits of `m` slices, in any order:
+// f(composite) for each, over all threads.  Eight loads at a time are in
+// flight per thread (one after the other, 20 slices took 10 us).
+template <class F>
+QM_DEV void for_slices(const SampleArgs& A, const int* list, int m, bool tie_last, F f) {
+    const int shift = 31 - __builtin_clz(A.chunk), total = m << shift;   // chunk is a power of two
+    for (int i0 = threadIdx.x; i0 < total; i0 += 8 * SMP_THREADS) {
+        int id[8];
+        float l[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int i = min(i0 + u * SMP_THREADS, total - 1);
+            id[u] = (list[i >> shift] << shift) + (i & (A.chunk - 1));
+            l[u] = A.logits[min(id[u], A.vocab - 1)];
+            if (i0 + u * SMP_THREADS >= total) id[u] = A.vocab;
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (id[u] < A.vocab) f(cand_pack(logit_key(l[u]), id[u], tie_last));
+    }
+}
+
+// The selection over qm_sample_slices' keys, and the draw, for k <= 64 and
+// at least k slices (see the head of this file).
+extern "C" __global__ __launch_bounds__(SMP_THREADS) void qm_sample_draw(SampleArgs A) {
+#pragma clang fp contract(off)
+    __shared__ uint32_t smax[SMP_MAX_LISTS];
+    __shared__ int list[SMP_MAX_LISTS];
+    __shared__ uint64_t cand[SMP_DRAW_CAND];
+    __shared__ uint64_t top[64];
+    __shared__ uint32_t hist[256], pick[2];
+    __shared__ uint32_t bound, nlist, ncand;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const bool greedy = !(A.temperature > 0.0f);
+    const int k = greedy ? 1 : min(A.top_k, A.vocab);
+    const bool tie_last = greedy && (A.flags & QMK_SAMPLE_WGPU);
+    const int ns = (A.vocab + A.chunk - 1) / A.chunk;
+    // the generator's state is needed last and requested first
+    const uint64_t rng = tid < 64 && !greedy ? A.rng_state[0] : 0;
+    if (tid < SMP_MAX_LISTS) smax[tid] = tid < ns ? reinterpret_cast<const uint32_t*>(A.cand)[tid] : 0u;
+    if (tid == 0) nlist = ncand = 0;
+    __syncthreads();
+    // the k-th largest slice maximum: at least k logits reach it.  Four
+    // threads per slice count the larger ones (equal ones by index).
+    {
+        const int i = tid >> 2;
+        const uint32_t mine = smax[i];
+        int above = 0;
+#pragma unroll 4
+        for (int j = 4 * (tid & 3); j < SMP_MAX_LISTS; j += 16) {   // zeros past ns
+            const uint4 o = *reinterpret_cast<const uint4*>(&smax[j]);
+            above += (o.x > mine || (o.x == mine && j < i)) + (o.y > mine || (o.y == mine && j + 1 < i)) +
+                     (o.z > mine || (o.z == mine && j + 2 < i)) + (o.w > mine || (o.w == mine && j + 3 < i));
+        }
+        above += __shfl_xor(above, 1);
+        above += __shfl_xor(above, 2);
+        if (i < ns && (tid & 3) == 0 && above == k - 1) bound = mine;
+    }
+    __syncthreads();
+    if (tid < ns && smax[tid] >= bound) list[atomicAdd(&nlist, 1u)] = tid;
+    __syncthreads();
+    const int m = (int)nlist;
+    const uint64_t floor = (uint64_t)bound << 32;
+    for_slices(A, list, m, tie_last, [&](uint64_t c) {
+        if (c < floor) return;
+        const uint32_t slot = atomicAdd(&ncand, 1u);
+        if (slot < SMP_DRAW_CAND) cand[slot] = c;
+    });
+    __syncthreads();
+    int n = (int)ncand;
+    if (n > SMP_DRAW_CAND) {
+        // More logits reach the bound than are ranked by counting (thousands
+        // of equal ones, or a slice of nothing but large ones): the k-th
+        // largest composite by radix select, eight digits of eight bits.
+        // Composites are distinct, so exactly k reach it.
+        uint64_t prefix = 0, mask = 0;
+        uint32_t rank = (uint32_t)k;
+        for (int shift = 56; shift >= 0; shift -= 8) {
+            __syncthreads();
+            if (tid < 256) hist[tid] = 0;
+            __syncthreads();
+            for_slices(A, list, m, tie_last, [&](uint64_t c) {
+                if (c < floor || (c & mask) != prefix) return;
+                const uint32_t d = (uint32_t)(c >> shift) & 255u;
+                // equal logits share their upper digits: one add per wave then
+                const uint64_t on = __ballot(1);
+                if (__ballot(d == (uint32_t)__builtin_amdgcn_readfirstlane((int)d)) == on) {
+                    if (lane == __builtin_ctzll(on)) atomicAdd(&hist[d], (uint32_t)__popcll(on));
+                } else {
+                    atomicAdd(&hist[d], 1u);
+                }
+            });
+            __syncthreads();
+            if (tid < 64) radix_pick(hist, rank, pick);
+            __syncthreads();
+            prefix |= (uint64_t)pick[0] << shift;
+            rank -= pick[1];
+            mask |= 255ull << shift;
+        }
+        if (tid == 0) ncand = 0;
+        __syncthreads();
+        for_slices(A, list, m, tie_last, [&](uint64_t c) {
+            if (c >= prefix) cand[atomicAdd(&ncand, 1u)] = c;
+        });
+        __syncthreads();
+        n = k;
+    }
+    // rank by counting (n is a few times k), eight threads per candidate
+    for (int i0 = 0; i0 < n; i0 += SMP_THREADS / 8) {
+        const int i = i0 + (tid >> 3);
+        const uint64_t mine = cand[min(i, n - 1)];
+        int above = 0;
+#pragma unroll 4
+        for (int j = tid & 7; j < n; j += 8) above += cand[j] > mine;
+        above += __shfl_xor(above, 1);
+        above += __shfl_xor(above, 2);
+        above += __shfl_xor(above, 4);
+        if (i < n && (tid & 7) == 0 && above < k) top[above] = mine;
+    }
+    __syncthreads();
+    if (tid >= 64) return;
+    const uint64_t c = lane < k ? top[lane] : 0;
+    const int32_t id = cand_id(c, tie_last), best = __builtin_amdgcn_readlane(id, 0);
+    if (A.top_ids && lane < k) A.top_ids[lane] = id;
+    if (greedy) {                      // generate.rs:335-342 (first maximum; last for the wgpu twin)
+        if (lane == 0) A.token_out[0] = best;
+        return;
+    }
+    // generate.rs:345-383 as in qm_sample_top_k, in the reference's order
+    // and rounding.  Its cutoff, total and draw loops all add the same
+    // probabilities from zero: one running sum, lane i keeping the i-th.
+    const float inv_temp = __fdiv_rn(1.0f, A.temperature);
+    const float l = key_logit((uint32_t)(c >> 32));
+    float p = (float)exp((double)__fmul_rn(__fsub_rn(l, readlane_f32(l, 0)), inv_temp));
+    float sum = 0.0f;
+    for (int i = 0; i < k; ++i) sum = __fadd_rn(sum, readlane_f32(p, i));
+    const bool wgpu = A.flags & QMK_SAMPLE_WGPU;
+    if (!wgpu && sum <= 0.0f) {
+        if (lane == 0) A.token_out[0] = best;
+        return;
+    }
+    p = wgpu ? __fdiv_rn(p, sum) : __fmul_rn(p, __fdiv_rn(1.0f, sum));
+    if (A.top_probs && lane < k) A.top_probs[lane] = p;
+    float run = 0.0f, upto = 0.0f;
+    for (int i = 0; i < k; ++i) {
+        run = __fadd_rn(run, readlane_f32(p, i));
+        upto = lane == i ? run : upto;
+    }
+    const uint64_t reach = __ballot(lane < k && upto >= A.top_p);
+    const int cutoff = reach ? __builtin_ctzll(reach) + 1 : k;
+    const float total = readlane_f32(upto, cutoff - 1);
+    if (!wgpu && total <= 0.0f) {
+        if (lane == 0) A.token_out[0] = best;
+        return;
+    }
+    // Rng::next_f32, generate.rs:46-54
+    uint64_t s = rng;
+    s ^= s << 13;
+    s ^= s >> 7;
+    s ^= s << 17;
+    const float rand_val = __fmul_rn((float)(uint32_t)(s >> 40) / 16777216.0f, total);
+    const uint64_t hit = __ballot(lane < cutoff && upto >= rand_val);
+    const int32_t tok = hit ? __builtin_amdgcn_readlane(id, __builtin_ctzll(hit)) : best;
+    if (lane == 0) {
+        A.rng_state[0] = s;
+        A.token_out[0] = tok;
+    }
 }

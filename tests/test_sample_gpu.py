@@ -76,6 +76,45 @@ def test_sample_all_equal_and_small_vocab(ctx):
     assert int(ctx.download(dst, (1,), np.uint64)[0]) == int(st[0])
 
 
+# The short way (k <= 64 of at least k slices of 1024, 512 or 256 logits) at
+# its edges: exactly k slices of each size and one logit fewer (the general
+# way), one slice per draw at 256 slices, and logits whose largest values sit
+# together, so that thousands reach the bound the slice maxima give.
+@pytest.mark.parametrize("vocab,top_k,shape", [
+    (262144, 64, "normal"), (20 * 1024, 20, "normal"), (19 * 1024 + 1, 20, "normal"), (20 * 512, 20, "normal"),
+    (19 * 256 + 1, 20, "normal"), (19 * 256, 20, "normal"), (64 * 256 - 255, 64, "tied"), (300, 1, "tied"),
+    (100003, 33, "sorted"), (100003, 64, "two levels"), (50000, 20, "tied")])
+def test_sample_slices(ctx, vocab, top_k, shape):
+    rng = np.random.default_rng(vocab + top_k)
+    x = (3.0 * rng.standard_normal(vocab)).astype(np.float32)
+    if shape == "tied":
+        x = (np.round(x) / 2).astype(np.float32)
+    elif shape == "sorted":
+        x = np.sort(x)[::-1].copy()
+    elif shape == "two levels":                           # one block of 6000 equal logits over the rest
+        x[7000:13000] = 20.0
+    gen = rng.integers(0, vocab, 500).astype(np.int32)
+    gen[-30:-10] = np.argsort(-x, kind="stable")[:20]     # penalties move the candidates
+    gen[-5:] = gen[-30]
+    for temp, wgpu in ((0.9, False), (0.9, True), (0.0, False), (0.0, True)):
+        want_x = O.apply_penalties(x, gen, 1.1, 0.5)
+        banned = int(np.argmax(want_x))
+        want_x[banned] = -np.inf
+        dx, dg, dst = ctx.upload(x), ctx.upload(gen), ctx.upload(np.array([vocab], np.uint64))
+        k = 1 if temp <= 0 else top_k
+        tok, ids = ctx.alloc(4), ctx.alloc(4 * k)
+        st = np.array([vocab], np.uint64)
+        print(f"case: sample slices vocab={vocab} k={top_k} {shape} T={temp} wgpu={wgpu}", flush=True)
+        ctx.sample(vocab, dx, dg, len(gen), dst, tok, temperature=temp, top_p=0.98, top_k=top_k,
+                   repetition_penalty=1.1, presence_penalty=0.5, banned_id=banned,
+                   flags=M.QM_SAMPLE_WGPU if wgpu else 0, top_ids=ids)
+        want, wids, _ = O.sample_top_k(want_x, temp, 0.98, top_k, st, wgpu=wgpu)
+        assert np.array_equal(ctx.download(dx, (vocab,), np.float32), want_x)
+        assert np.array_equal(ctx.download(ids, (k,), np.int32), wids[:k])
+        assert int(ctx.download(tok, (1,), np.int32)[0]) == want
+        assert int(ctx.download(dst, (1,), np.uint64)[0]) == int(st[0])
+
+
 def test_penalties_in_place(ctx):
     """generate.rs:58-82 then the think-block EOS ban (generate.rs:191)."""
     rng = np.random.default_rng(5)
