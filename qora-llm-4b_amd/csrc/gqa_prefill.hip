@@ -201,10 +201,14 @@ extern "C" __global__ __launch_bounds__(512) void qm_gqa_prefill_kv(GqaPrefillAr
 #define SM_V(b) ((b) * 65536 + 32768)
 #define SM_BYTES 131072
 
-// A row block is 48 query rows of the four query heads of one kv group: 12
-// waves, wave w on head 4g + (w & 3) and rows 16 (w >> 2) .. +15, three
-// waves per SIMD, so one wave's LDS and softmax latency hides behind the
-// other waves' MFMAs.  Each iteration fetches the next K / V^T tile by LDS
+// A row block is 16 R query rows of the four query heads of one kv group: 4 R
+// waves, wave w on head 4g + (w & 3) and rows 16 (w >> 2) .. +15.  R = 3 puts
+// three waves on a SIMD, so one wave's LDS and softmax latency hides behind
+// the other waves' MFMAs; R = 2 makes half as many blocks again and each a
+// third shorter, for prompts whose blocks do not fill the CUs otherwise (the
+// host's rule: the whole call at 700 tokens 42.7 -> 34.8 us, 2048 83.4 ->
+// 70.3).  A row's arithmetic does not depend on R: the outputs are the same
+// bits.  Each iteration fetches the next K / V^T tile by LDS
 // DMA (the tile's 64 blocks dealt round-robin over the waves), then computes
 // the current tile's scores, softmax and P V.
 // The kernel is persistent: one workgroup per CU, workgroup b serving kv
@@ -217,7 +221,6 @@ extern "C" __global__ __launch_bounds__(512) void qm_gqa_prefill_kv(GqaPrefillAr
 // n-th longest block.  A workgroup whose own queue is empty takes the
 // remaining (short) blocks of the other groups, which evens out the XCDs'
 // speeds.
-#define TQ3 48
 
 // Fragment reads in flight per wave in the two products: with 32 reads of
 // 1 KB per product and three waves per SIMD, keeping 6 in flight (24 VGPRs)
@@ -238,13 +241,16 @@ QM_DEV void sched_reads_ahead() {
     __builtin_amdgcn_sched_group_barrier(0x008, LOOKAHEAD + EXTRA, 0);
 }
 
-extern "C" __global__ __launch_bounds__(768) void qm_gqa_prefill_attn(GqaPrefillAttnArgs P) {
+// R row groups of 16 rows: a row block of 16 R rows on 4 R waves.
+template <int R>
+QM_DEV void gqa_prefill_attn_body(const GqaPrefillAttnArgs& P) {
+    constexpr int TQ = 16 * R, NW = 4 * R;
     const GqaPrefillArgs& A = P.a;
     __shared__ __attribute__((aligned(1024))) char sm[SM_BYTES];
     __shared__ int item_s;
     const int tid = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nblk = (A.S + TQ3 - 1) / TQ3;
+    const int nblk = (A.S + TQ - 1) / TQ;
     const uint32_t sm_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)sm;
     // item = group * nblk + block index; own group first, then the others
     // (the own group's index may already have been drawn: first)
@@ -276,19 +282,19 @@ extern "C" __global__ __launch_bounds__(768) void qm_gqa_prefill_attn(GqaPrefill
         const int lr = lane & 15, lq = lane >> 4;
         const int draw = item - g * nblk;
         const int tb = P.ordered ? (int)P.order[draw] : nblk - 1 - draw;
-        const int t0 = tb * TQ3;
+        const int t0 = tb * TQ;
         const int qh = 4 * g + (w & 3);
         const int r0 = t0 + 16 * (w >> 2);
         // tiles up to the block's last row, within the zero-padded V^T copy
-        const int nkt = min((t0 + TQ3 + KT - 1) / KT, A.s_pad / KT);
+        const int nkt = min((t0 + TQ + KT - 1) / KT, A.s_pad / KT);
 
         // tile fetch, K half (blocks 0..31) or V^T half (32..63): block
-        // h + w + 12 j, one contiguous 1 KB piece each
+        // h + w + NW j, one contiguous 1 KB piece each
         auto fetch = [&](int kt, int buf, int h) {
             const uint16_t* src = tiles + (size_t)kt * (64 * 512) + 8 * lane;
 #pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                const int b = h + w + 12 * j;
+            for (int j = 0; j < (32 + NW - 1) / NW; ++j) {
+                const int b = h + w + NW * j;
                 if (b < h + 32) dma16(src + 512 * b, sm_lds + SM_K(buf) + 1024 * b);
             }
         };
@@ -503,3 +509,6 @@ extern "C" __global__ __launch_bounds__(768) void qm_gqa_prefill_attn(GqaPrefill
         item = item_s;
     }
 }
+
+extern "C" __global__ __launch_bounds__(768) void qm_gqa_prefill_attn(GqaPrefillAttnArgs P) { gqa_prefill_attn_body<3>(P); }
+extern "C" __global__ __launch_bounds__(512) void qm_gqa_prefill_attn_r2(GqaPrefillAttnArgs P) { gqa_prefill_attn_body<2>(P); }

@@ -46,7 +46,7 @@ struct qm_context {
     hipFunction_t f_dnp_scan = nullptr;
     hipFunction_t f_dnp_out = nullptr;
     hipFunction_t f_gqp_kv = nullptr;
-    hipFunction_t f_gqp_attn = nullptr;
+    hipFunction_t f_gqp_attn[2] = {};        // row blocks of 32 and of 48 rows
     hipFunction_t f_q4_gemv = nullptr;
     hipFunction_t f_q4_gemv_hidden = nullptr;  // k <= 2560 (the hidden size)
     hipFunction_t f_q4_gemv_inter = nullptr;   // 4096 < k <= 9216 (the MLP's intermediate size)
@@ -359,7 +359,8 @@ int32_t qm_create(qm_context** out, const qm_config* cfg, const char* code_objec
     if (st == QM_OK) st = load_function(c, mods[3], "qm_dn_prefill_scan", &c->f_dnp_scan);
     if (st == QM_OK) st = load_function(c, mods[3], "qm_dn_prefill_out", &c->f_dnp_out);
     if (st == QM_OK) st = load_function(c, mods[4], "qm_gqa_prefill_kv", &c->f_gqp_kv);
-    if (st == QM_OK) st = load_function(c, mods[4], "qm_gqa_prefill_attn", &c->f_gqp_attn);
+    if (st == QM_OK) st = load_function(c, mods[4], "qm_gqa_prefill_attn_r2", &c->f_gqp_attn[0]);
+    if (st == QM_OK) st = load_function(c, mods[4], "qm_gqa_prefill_attn", &c->f_gqp_attn[1]);
     if (st == QM_OK) st = load_function(c, mods[5], "qm_q4_gemv", &c->f_q4_gemv);
     if (st == QM_OK) st = load_function(c, mods[5], "qm_q4_gemv_hidden", &c->f_q4_gemv_hidden);
     if (st == QM_OK) st = load_function(c, mods[5], "qm_q4_gemv_inter", &c->f_q4_gemv_inter);
@@ -864,10 +865,23 @@ int32_t qm_gqa_prefill(qm_context* c, qm_stream stream, int32_t seq_len, const u
     st = launch(c, c->f_gqp_kv, static_cast<uint32_t>(s_pad / 64) * QM_GQA_KV_HEADS, c->gqp_kv_threads, ga, s,
                 "qm_gqa_prefill_kv");
     if (st != QM_OK) return st;
+    // Row blocks of 32 rows (8 waves) up to 4400 tokens, where blocks of 48
+    // (12 waves) leave CUs idle or the longest block's chain of tiles bounds
+    // the call; above, a tile's fetch feeding twelve waves is worth more.
+    // Measured, us, 32 / 48: 300 tokens 25.2 / 30.6, 700 34.8 / 42.7, 2048
+    // 70.3 / 83.4, 3000 101 / 123, 4200 169 / 178, 4400 183 / 187, 4600
+    // 198 / 196, 5000 235 / 225 (blocks of 16: 27.7, 42.8, 107, 208).  A
+    // forced packed order is a plan of 48-row blocks.
+    const int32_t groups = seq_len <= 4400 && c->opt_gqp_order != 2 ? 2 : 3;
     // persistent: one workgroup per CU (a multiple of the 4 kv groups), no
-    // more than there are 48-row blocks
-    const int32_t nblk = (seq_len + 47) / 48;
+    // more than there are row blocks
+    const int32_t nblk = (seq_len + 16 * groups - 1) / (16 * groups);
     const int32_t per_group = std::max(1, std::min(c->num_cu / QM_GQA_KV_HEADS, nblk));
+    c->gqp_args.a = ga;
+    c->gqp_args.ordered = 0;
+    if (groups == 2)
+        return launch(c, c->f_gqp_attn[0], static_cast<uint32_t>(per_group) * QM_GQA_KV_HEADS, 512, c->gqp_args, s,
+                      "qm_gqa_prefill_attn_r2");
     qm_context::GqpPlan* plan = nullptr;
     for (auto& p : c->gqp_plans)
         if (p.S == seq_len && p.bins == per_group && p.mode == c->opt_gqp_order) plan = &p;
@@ -883,9 +897,8 @@ int32_t qm_gqa_prefill(qm_context* c, qm_stream stream, int32_t seq_len, const u
     plan->used = ++c->gqp_clock;
     c->gqp_args.ordered = plan->ordered;
     if (plan->ordered)
-        std::memcpy(c->gqp_args.order, plan->order, sizeof(uint16_t) * static_cast<size_t>((seq_len + 47) / 48));
-    c->gqp_args.a = ga;
-    return launch(c, c->f_gqp_attn, static_cast<uint32_t>(per_group) * QM_GQA_KV_HEADS, 768, c->gqp_args,
+        std::memcpy(c->gqp_args.order, plan->order, sizeof(uint16_t) * static_cast<size_t>(nblk));
+    return launch(c, c->f_gqp_attn[1], static_cast<uint32_t>(per_group) * QM_GQA_KV_HEADS, 768, c->gqp_args,
                   s, "qm_gqa_prefill_attn");
 }
 

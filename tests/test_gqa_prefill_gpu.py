@@ -95,6 +95,20 @@ def test_prefill_5000_rows(ctx):
     check(o, K, V, ref, kc, vc, rows)
 
 
+@pytest.mark.parametrize("S", [33, 1057, 4400, 4401])
+def test_prefill_row_block_forms(ctx, S):
+    """32-row blocks up to 4400 tokens, 48-row ones above: a last block of one
+    row (33, 1057), the last length of the one form and the first of the
+    other, on the first, last and random rows."""
+    w = W.gqa_prefill_workload(S, seed=29 + S)
+    print(f"case: gqa prefill row block forms S={S}", flush=True)
+    o, K, V = run_gpu(ctx, w, S, S + 1)
+    rows = np.unique(np.concatenate([np.arange(0, min(S, 34)), np.arange(max(0, S - 50), S),
+                                     np.random.default_rng(S).integers(0, S, 60)]))
+    ref, kc, vc = run_oracle(w, S, rows=rows)
+    check(o, K, V, ref, kc, vc, rows)
+
+
 @pytest.mark.parametrize("S", [8192, 10000, 5000])
 def test_prefill_block_order(ctx, S):
     """The packed row-block order (QM_OPT_GQA_PREFILL_ORDER = 2; at 8192 and
