@@ -64,6 +64,22 @@ def test_lm_head_shapes(ctx, vocab, hidden):
     assert np.all(np.abs(got - ref) <= 1e-5 * mag)
 
 
+@pytest.mark.parametrize("vocab,hidden,power", [(3 * 256 * 32 + 33, 2560, -80), (256 * 32 + 1, 8192, 80)])
+def test_lm_head_rows_per_workgroup_and_range(ctx, vocab, hidden, power):
+    """One row more than the grid takes in whole rounds (256 CUs), within the
+    bar of the oracle; and x times a power of two gives the logits times it,
+    bit for bit: the factors that let the codes enter as f16 subnormals come
+    out again."""
+    rng, packed, scales = _embed(vocab, hidden, vocab)
+    x = rng.standard_normal(hidden).astype(np.float32)
+    print(f"case: lm_head {vocab} x {hidden}, x * 2^{power}", flush=True)
+    got = _lm_head(ctx, x, None, packed, scales)
+    ref = O.q4_lm_head(x, packed, scales).astype(np.float64)
+    mag = np.abs(W.q4_dequant(packed, scales)).astype(np.float64) @ np.abs(x).astype(np.float64)
+    assert np.all(np.abs(got.astype(np.float64) - ref) <= 1e-5 * mag)
+    assert np.array_equal(_lm_head(ctx, np.ldexp(x, power), None, packed, scales), np.ldexp(got, power))
+
+
 def test_embed_rows_exact(ctx):
     vocab, hidden = 248320, 2560
     _, packed, scales = _embed(vocab, hidden, 82)
