@@ -32,12 +32,16 @@
 // rows so that no load waits behind a branch.  The T partial sums of every
 // lane are reduced across the wave in registers (a transpose-reduce over
 // lane swaps), then across the waves through LDS behind one barrier, in a
-// fixed order (bit-reproducible run to run).  Dequantization costs ~2.4 VALU ops per weight: the codes are split
-// into low and high nibble bytes by two masks, each byte converts with one
-// v_cvt_f32_ubyteN, and the fma uses q itself, the -8 offset being applied
-// once per lane through sum(scale * x).  The RMSNorm is applied by
-// linearity: y = inv_rms * (x (1 + gamma)) W, so its sum of squares comes
-// from the same x loads and the factor scales the column sums.
+// fixed order (bit-reproducible run to run).  A weight costs ~1.7 VALU
+// instructions: the codes enter the fma as f16 (see q4_halves) and as q
+// itself, the -8 offset being applied once per lane through sum(scale * x).
+// (With a v_cvt_f32_ubyteN per code, 2.4 instructions, the four launches of
+// a layer took 0.4 us more: 2560 x 12288 6.45 -> 6.31 us, 9216 x 2560 7.15
+// -> 7.02, 4096 x 2560 4.35 -> 4.26, the gate / up pair unchanged at 9.7,
+// of which 1.9 are an empty launch and 4.3 the weights at 6.2 TB/s.)
+// The RMSNorm is applied by linearity: y = inv_rms * (x (1 + gamma)) W, so
+// its sum of squares comes from the same x loads and the factor scales the
+// column sums.
 #include "qm_device.h"
 #include "qm_q4_tiles.h"
 #include <type_traits>
@@ -59,19 +63,19 @@ template <> struct Q4Pair<8> {
     static QM_DEV uint32_t half(uint2 v, int h) { return h ? v.y : v.x; }
 };
 
-QM_DEV void q4_word(float* acc, uint32_t w, float sx) {  // 8 codes: columns 0..7 of acc
-    uint32_t lo = w & 0x0f0f0f0fu, hi = (w >> 4) & 0x0f0f0f0fu;
-    // opaque to the optimiser, which would otherwise fold each mask into a
-    // per-nibble bit-field extract (one more op each)
-    asm volatile("" : "+v"(lo), "+v"(hi));
+QM_DEV void q4_word(float* acc, uint32_t w, float se, float so) {  // 8 codes: columns 0..7 of acc
+    q4_half2 h[4];
+    q4_halves(w, h);
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-        acc[2 * b] = fmaf((float)((lo >> (8 * b)) & 0xffu), sx, acc[2 * b]);
-        acc[2 * b + 1] = fmaf((float)((hi >> (8 * b)) & 0xffu), sx, acc[2 * b + 1]);
-    }
+    for (int b = 0; b < 8; ++b) acc[b] = fmaf((float)h[b & 3][b >> 2], b & 1 ? so : se, acc[b]);
 }
-QM_DEV void q4_accumulate(float (&acc)[16], uint2 c, float sx) { q4_word(acc, c.x, sx); q4_word(acc + 8, c.y, sx); }
-QM_DEV void q4_accumulate(float (&acc)[8], uint32_t c, float sx) { q4_word(acc, c, sx); }
+// acc += q * sx / QM_Q4_SUM
+QM_DEV void q4_accumulate(float (&acc)[16], uint2 c, float sx) {
+    const float se = sx * QM_Q4_EVEN, so = sx * QM_Q4_ODD;
+    q4_word(acc, c.x, se, so);
+    q4_word(acc + 8, c.y, se, so);
+}
+QM_DEV void q4_accumulate(float (&acc)[8], uint32_t c, float sx) { q4_word(acc, c, sx * QM_Q4_EVEN, sx * QM_Q4_ODD); }
 
 // Wave-level sum of each of a lane's T column partials by transpose-reduce:
 // each step pairs lane l with l ^ 32, ^16, ^8 (and ^4 for T = 16), and each
@@ -256,12 +260,12 @@ QM_DEV void q4_tile(const Q4GemvArgs& A, int p, int tile, float (*red)[33]) {
     // waves' values in order.  x's sum of squares for the RMSNorm rides along.
     const int lane = tid & 63, wv = tid >> 6;
 #pragma unroll
-    for (int j = 0; j < T; ++j) acc[j] = fmaf(-8.0f, bsum, acc[j]);
+    for (int j = 0; j < T; ++j) acc[j] = fmaf(QM_Q4_SUM, acc[j], -8.0f * bsum);
     const float cs = q4_wave_reduce<T>(acc, lane);
     float cs_u = 0.0f;
     if (GATE_UP) {
 #pragma unroll
-        for (int j = 0; j < T; ++j) acc_u[j] = fmaf(-8.0f, bsum_u, acc_u[j]);
+        for (int j = 0; j < T; ++j) acc_u[j] = fmaf(QM_Q4_SUM, acc_u[j], -8.0f * bsum_u);
         cs_u = q4_wave_reduce<T>(reinterpret_cast<float(&)[T]>(acc_u), lane);
     }
     const float ssw = NORM ? wave_sum64(ss) : 0.0f;
@@ -339,7 +343,7 @@ extern "C" __global__ __launch_bounds__(Q4_THREADS) void qm_q4_gemv(Q4GemvArgs A
 }
 
 // 256 threads, 10 rows (5 row pairs) per lane: one load round at k = 2560,
-// and at 132 VGPRs three workgroups per CU, so the 576 tiles of the 2560 x
+// and at 140 VGPRs three workgroups per CU, so the 576 tiles of the 2560 x
 // 9216 gate / up pair are resident in one dispatch round (the 512-thread form
 // fitted two per CU and ran 3% slower per model token).
 extern "C" __global__ __launch_bounds__(256) void qm_q4_gate_up(Q4GemvArgs A) {
@@ -349,11 +353,11 @@ extern "C" __global__ __launch_bounds__(256) void qm_q4_gate_up(Q4GemvArgs A) {
 // Shape-fitted forms.  A launch's workgroups should all be resident at once
 // (a second dispatch round repeats the whole load -> reduce latency), and a
 // lane's rows should come in as few load rounds as possible:
-//   k <= 2560 (the hidden size): 256 threads of 10 rows, one load round, 84
+//   k <= 2560 (the hidden size): 256 threads of 10 rows, one load round, 87
 //     VGPRs (five workgroups per CU, 1280 slots for the 776 tiles of the
 //     fused DeltaNet input projections);
 //   k <= 9216 without a norm (the MLP's down_proj): 18 rows per lane, one
-//     load round, 115 VGPRs (two workgroups per CU, 512 slots for 320
+//     load round, 116 VGPRs (two workgroups per CU, 512 slots for 320
 //     tiles); the host sends a launch with a norm to the general form.
 // (512-thread forms of 5 rows for k <= 2560, of 18 or 12 rows at 256 threads
 // for down_proj, and of 16 at 256 threads for the general case all measured

@@ -17,7 +17,7 @@
 // logit = inv_rms * (x (1 + gamma)) . row, with inv_rms from the lanes' own
 // x slices.  Dequantization: the -8 code offset is applied once per group
 // through the group's sum of x, and the codes enter the fma as f16 (see
-// q4_word_dot), 1.6 instructions a weight: with a conversion per code, 2.4, the
+// q4_halves), 1.6 instructions a weight: with a conversion per code, 2.4, the
 // arithmetic alone took 39 us of the 358 MB stream's 58.
 //
 // qm_q4_embed: x[t] = row ids[t] dequantized (embed_lookup_q4,
@@ -26,31 +26,14 @@
 #include "qm_device.h"
 #include "qm_kernel_args.h"
 
-// A 4-bit code q in the low bits of a 16-bit half is the f16 subnormal
-// q * 2^-24, and in bits 4..7 it is q * 2^-20, both exact: a word's 8 codes
-// become f16 operands by four masks and one shift, and v_fma_mix_f32 takes
-// either half straight into an f32 fma (13 instructions for 8 codes against
-// 19 with a v_cvt_f32_ubyteN per code).  The factors go into the f32 side: x
-// of an even column times Q4_EVEN, of an odd one times Q4_ODD, and the sum
-// times Q4_SUM, all powers of two, so the results are the same bits as with
-// the codes converted (half of the 2^24 is put on each side of the sum, so
-// that neither end of f32's range comes near).
-#define Q4_EVEN 4096.0f
-#define Q4_ODD 256.0f
-#define Q4_SUM 4096.0f
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-
 // 8 codes (one 32-bit word: columns 8t .. 8t + 7 of a group) against the
-// matching scaled x values; returns the sum of q * x over them / Q4_SUM.
+// matching x values (scaled by QM_Q4_EVEN / QM_Q4_ODD); returns the sum of
+// q * x over them / QM_Q4_SUM.
 QM_DEV float q4_word_dot(uint32_t w, const float* xw, float acc) {
-    const uint32_t v = w >> 8;
-    uint32_t m[4] = {w & 0x000f000fu, w & 0x00f000f0u, v & 0x000f000fu, v & 0x00f000f0u};
-    // keep the masks: the optimiser would otherwise fold each into a
-    // per-nibble bit-field extract
-    asm volatile("" : "+v"(m[0]), "+v"(m[1]), "+v"(m[2]), "+v"(m[3]));
+    q4_half2 h[4];
+    q4_halves(w, h);
 #pragma unroll
-    for (int b = 0; b < 8; ++b)                 // m[i] holds columns i and i + 4
-        acc = fmaf((float)__builtin_bit_cast(half2_t, m[b & 3])[b >> 2], xw[b], acc);
+    for (int b = 0; b < 8; ++b) acc = fmaf((float)h[b & 3][b >> 2], xw[b], acc);
     return acc;
 }
 
@@ -116,8 +99,8 @@ extern "C" __global__ __launch_bounds__(1024) void qm_q4_lm_head(LmHeadArgs A) {
     sx *= 8.0f;
 #pragma unroll
     for (int e = 0; e < 32; e += 2) {
-        xs[e] *= Q4_EVEN;
-        xs[e + 1] *= Q4_ODD;
+        xs[e] *= QM_Q4_EVEN;
+        xs[e + 1] *= QM_Q4_ODD;
     }
 
     const int nsb = (A.vocab + 4 * LMH_SB - 1) / (4 * LMH_SB);
@@ -139,7 +122,7 @@ extern "C" __global__ __launch_bounds__(1024) void qm_q4_lm_head(LmHeadArgs A) {
             d = q4_word_dot(c[b].y, &xs[8], d);
             d = q4_word_dot(c[b].z, &xs[16], d);
             d = q4_word_dot(c[b].w, &xs[24], d);
-            const float p = row_sum16(f16_to_f32(sc[b]) * fmaf(d, Q4_SUM, -sx));
+            const float p = row_sum16(f16_to_f32(sc[b]) * fmaf(d, QM_Q4_SUM, -sx));
             if (sl == 0) part[b][seg] = p;
         }
         __syncthreads();

@@ -69,6 +69,31 @@ QM_DEV float wave_sum64(float x) {
 QM_DEV float f16_to_f32(uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
 QM_DEV uint16_t f32_to_f16(float f) { return __builtin_bit_cast(uint16_t, (_Float16)f); }
 QM_DEV float bf16_to_f32(uint16_t h) { return __builtin_bit_cast(float, (uint32_t)h << 16); }
+// ---- Q4 codes as f16 ------------------------------------------------------
+// A 4-bit code q in the low bits of a 16-bit half is the f16 subnormal
+// q * 2^-24, and in bits 4..7 it is q * 2^-20, both exact: a word's 8 codes
+// become f16 operands by four masks and one shift, and v_fma_mix_f32 takes
+// either half straight into an f32 fma (13 instructions for 8 codes against
+// 19 with a v_cvt_f32_ubyteN per code).  The factors go into the f32 side:
+// the operand of an even column times QM_Q4_EVEN, of an odd one times
+// QM_Q4_ODD, and the sum times QM_Q4_SUM, all powers of two, so the results
+// are the same bits as with the codes converted (half of the 2^24 is put on
+// each side of the sum, so that neither end of f32's range comes near).
+#define QM_Q4_EVEN 4096.0f
+#define QM_Q4_ODD 256.0f
+#define QM_Q4_SUM 4096.0f
+typedef _Float16 q4_half2 __attribute__((ext_vector_type(2)));
+// h[i] holds columns i and i + 4 of the word
+QM_DEV void q4_halves(uint32_t w, q4_half2 (&h)[4]) {
+    const uint32_t v = w >> 8;
+    uint32_t m[4] = {w & 0x000f000fu, w & 0x00f000f0u, v & 0x000f000fu, v & 0x00f000f0u};
+    // opaque to the optimiser, which would otherwise fold each mask into a
+    // per-nibble bit-field extract (one more op each)
+    asm volatile("" : "+v"(m[0]), "+v"(m[1]), "+v"(m[2]), "+v"(m[3]));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) h[i] = __builtin_bit_cast(q4_half2, m[i]);
+}
+
 // f32 -> bf16, round to nearest even: one v_cvt_pk_bf16_f32 (gfx950) per
 // pair of values, where the integer form (NaN test, bias, carry) took ~6
 // VALU ops per value.  NaN stays NaN.

@@ -65,6 +65,18 @@ def test_q4_gemv_ragged(ctx, k, n):
     check(run_gpu(ctx, w["x"], w["packed"], w["scales"]), w["x"], w["packed"], w["scales"])
 
 
+@pytest.mark.parametrize("k,n,power", [(37, 64, 80), (2560, 4096, -80), (5000, 2560, 80)])
+def test_q4_gemv_range(ctx, k, n, power):
+    """x times a power of two gives y times it, bit for bit (tiles of 8 and 16
+    columns, odd k): the factors that let the codes enter as f16 subnormals
+    come out again."""
+    w = W.q4_gemv_workload(k, n, seed=k)
+    print(f"case: q4 gemv k={k} n={n}, x * 2^{power}", flush=True)
+    got = run_gpu(ctx, w["x"], w["packed"], w["scales"])
+    scaled = run_gpu(ctx, np.ldexp(w["x"], power), w["packed"], w["scales"])
+    assert np.array_equal(scaled, np.ldexp(got, power))
+
+
 def test_q4_gemv_multi_layer_projections(ctx):
     """in_proj_qkv, in_proj_z, in_proj_a, in_proj_b of one input in one launch,
     each output as its own qm_q4_gemv would give it (bit for bit) and within
