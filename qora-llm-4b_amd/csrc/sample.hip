@@ -31,15 +31,21 @@
 //   qm_sample_slices: each workgroup applies the penalties to its slice of the
 //      vocabulary and writes the slice's largest key;
 //   qm_sample_draw (one workgroup): the k-th largest of those keys is a lower
-//      bound of the k-th largest logit, and only slices that reach it hold
-//      candidates, so some 20 slices are read instead of sorting each; the
-//      candidates are ranked by counting, and one wave draws, its lanes
+//      bound of the k-th largest logit, and only the k slices with the largest
+//      keys hold candidates, so k slices are read instead of sorting each; the
+//      candidates that reach the bound are ranked by counting where they are
+//      few (logits spread over the vocabulary) and cut down to k by radix
+//      select where they are many (large logits beside each other, equal
+//      ones, a vocabulary mostly masked), and one wave draws, its lanes
 //      holding the probabilities.
 // What bounded the longer way was its chain of steps, not bytes: penalties 4.8
 // us, select 11.8 (four radix passes, a scan and a sort per slice), merge and
 // draw 14.6 (20 rounds of a 64-lane maximum, then one thread's loads from
 // LDS); now 5.3 and 11.2 us (248,320 logits, top 20, presence penalty over 1000
-// ids).
+// ids).  The whole call in a replayed graph, us, longer / shorter way: spread
+// logits 28.8 / 14.5, sorted ones 29.0 / 22.6, all equal 30.3 / 26.8, all but
+// five masked 28.6 / 26.8; at top 64 57.3 / 25.4, 58.2 / 45.3, 60.8 / 48.7,
+// 55.6 / 48.7; 32,000 generated ids 65.8 / 36.1.
 #include "qm_device.h"
 #include "qm_kernel_args.h"
 
@@ -49,7 +55,12 @@
 #define SMP_MAX_LISTS 256          // stage-1 slices (vocabulary / 1024 at most)
 #define SMP_MAX_VOCAB 262144       // the presence bitmap in LDS (32 KB)
 #define SMP_MAX_SLICE 1024         // logits per workgroup of qm_sample_slices (256, 512 or 1024)
-#define SMP_DRAW_CAND 4096         // candidates qm_sample_draw ranks by counting
+#define SMP_DRAW_CAND 4096         // candidates of qm_sample_draw: k <= 64 threads x 64 logits
+// Candidates ranked by counting, a quadratic cost; above, radix select comes
+// first.  Whole call, us, counting / select (248,320 logits, top 20): 128
+// candidates 15.7 / 16.6, 224 16.5 / 17.6, 320 19.4 / 17.5, 512 24.9 / 17.7,
+// 1000 44.8 / 17.9, 4000 453 / 21.0; at top 64 they cross near 192.
+#define SMP_COUNT_CAND 256
 
 // Larger logit -> larger key; -0 == +0; NaN below every number.
 QM_DEV uint32_t logit_key(float v) {
@@ -443,16 +454,51 @@ QM_DEV void for_slices(const SampleArgs& A, const int* list, int m, bool tie_las
     }
 }
 
+// The k-th largest of the n distinct composites in LDS, by radix select of
+// eight-bit digits from the top, ended as soon as a digit's bin is taken
+// whole: exactly k of them are >= the value returned.  All threads call it.
+QM_DEV uint64_t kth_largest(const uint64_t* c, int n, int k, uint32_t* hist, uint32_t* pick) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    uint64_t prefix = 0, mask = 0;
+    uint32_t rank = (uint32_t)k;
+    for (int shift = 56; shift >= 0; shift -= 8) {
+        __syncthreads();
+        if (tid < 256) hist[tid] = 0;
+        __syncthreads();
+        for (int i = tid; i < n; i += SMP_THREADS) {
+            const uint64_t v = c[i];
+            if ((v & mask) != prefix) continue;
+            const uint32_t d = (uint32_t)(v >> shift) & 255u;
+            // near logits share their upper digits: one add per wave then
+            const uint64_t on = __ballot(1);
+            if (__ballot(d == (uint32_t)__builtin_amdgcn_readfirstlane((int)d)) == on) {
+                if (lane == __builtin_ctzll(on)) atomicAdd(&hist[d], (uint32_t)__popcll(on));
+            } else {
+                atomicAdd(&hist[d], 1u);
+            }
+        }
+        __syncthreads();
+        if (tid < 64) radix_pick(hist, rank, pick);
+        __syncthreads();
+        prefix |= (uint64_t)pick[0] << shift;
+        rank -= pick[1];
+        mask |= 255ull << shift;
+        if (hist[pick[0]] == rank) break;
+    }
+    return prefix;
+}
+
 // The selection over qm_sample_slices' keys, and the draw, for k <= 64 and
 // at least k slices (see the head of this file).
 extern "C" __global__ __launch_bounds__(SMP_THREADS) void qm_sample_draw(SampleArgs A) {
 #pragma clang fp contract(off)
-    __shared__ uint32_t smax[SMP_MAX_LISTS];
-    __shared__ int list[SMP_MAX_LISTS];
+    __shared__ __attribute__((aligned(16))) uint32_t smax[SMP_MAX_LISTS];
+    __shared__ int list[64];
     __shared__ uint64_t cand[SMP_DRAW_CAND];
+    __shared__ uint64_t tmax[SMP_THREADS];
     __shared__ uint64_t top[64];
     __shared__ uint32_t hist[256], pick[2];
-    __shared__ uint32_t bound, nlist, ncand;
+    __shared__ uint32_t bound, ncand;
     const int tid = threadIdx.x, lane = tid & 63;
     const bool greedy = !(A.temperature > 0.0f);
     const int k = greedy ? 1 : min(A.top_k, A.vocab);
@@ -460,11 +506,15 @@ extern "C" __global__ __launch_bounds__(SMP_THREADS) void qm_sample_draw(SampleA
     const int ns = (A.vocab + A.chunk - 1) / A.chunk;
     // the generator's state is needed last and requested first
     const uint64_t rng = tid < 64 && !greedy ? A.rng_state[0] : 0;
-    if (tid < SMP_MAX_LISTS) smax[tid] = tid < ns ? reinterpret_cast<const uint32_t*>(A.cand)[tid] : 0u;
-    if (tid == 0) nlist = ncand = 0;
+    // slices in the order that ties are taken in
+    if (tid < SMP_MAX_LISTS)
+        smax[tid] = tid < ns ? reinterpret_cast<const uint32_t*>(A.cand)[tie_last ? ns - 1 - tid : tid] : 0u;
+    if (tid == 0) ncand = 0;
     __syncthreads();
-    // the k-th largest slice maximum: at least k logits reach it.  Four
-    // threads per slice count the larger ones (equal ones by index).
+    // The first k slices by (maximum, order): the k-th one's maximum is a key
+    // that at least k logits reach, and a logit of any other slice comes
+    // after those k (equal ones stand in an earlier slice).  Four threads per
+    // slice count the slices before it.
     {
         const int i = tid >> 2;
         const uint32_t mine = smax[i];
@@ -477,58 +527,66 @@ extern "C" __global__ __launch_bounds__(SMP_THREADS) void qm_sample_draw(SampleA
         }
         above += __shfl_xor(above, 1);
         above += __shfl_xor(above, 2);
-        if (i < ns && (tid & 3) == 0 && above == k - 1) bound = mine;
+        if (i < ns && (tid & 3) == 0 && above < k) {
+            list[above] = tie_last ? ns - 1 - i : i;
+            if (above == k - 1) bound = mine;
+        }
     }
     __syncthreads();
-    if (tid < ns && smax[tid] >= bound) list[atomicAdd(&nlist, 1u)] = tid;
-    __syncthreads();
-    const int m = (int)nlist;
-    const uint64_t floor = (uint64_t)bound << 32;
-    for_slices(A, list, m, tie_last, [&](uint64_t c) {
-        if (c < floor) return;
-        const uint32_t slot = atomicAdd(&ncand, 1u);
-        if (slot < SMP_DRAW_CAND) cand[slot] = c;
-    });
-    __syncthreads();
-    int n = (int)ncand;
-    if (n > SMP_DRAW_CAND) {
-        // More logits reach the bound than are ranked by counting (thousands
-        // of equal ones, or a slice of nothing but large ones): the k-th
-        // largest composite by radix select, eight digits of eight bits.
-        // Composites are distinct, so exactly k reach it.
-        uint64_t prefix = 0, mask = 0;
-        uint32_t rank = (uint32_t)k;
-        for (int shift = 56; shift >= 0; shift -= 8) {
-            __syncthreads();
-            if (tid < 256) hist[tid] = 0;
-            __syncthreads();
-            for_slices(A, list, m, tie_last, [&](uint64_t c) {
-                if (c < floor || (c & mask) != prefix) return;
-                const uint32_t d = (uint32_t)(c >> shift) & 255u;
-                // equal logits share their upper digits: one add per wave then
-                const uint64_t on = __ballot(1);
-                if (__ballot(d == (uint32_t)__builtin_amdgcn_readfirstlane((int)d)) == on) {
-                    if (lane == __builtin_ctzll(on)) atomicAdd(&hist[d], (uint32_t)__popcll(on));
-                } else {
-                    atomicAdd(&hist[d], 1u);
-                }
-            });
-            __syncthreads();
-            if (tid < 64) radix_pick(hist, rank, pick);
-            __syncthreads();
-            prefix |= (uint64_t)pick[0] << shift;
-            rank -= pick[1];
-            mask |= 255ull << shift;
+    // at most 64 logits a thread
+    uint64_t m = 0;                        // the thread's largest
+    auto collect = [&](uint64_t from) {
+        for_slices(A, list, k, tie_last, [&](uint64_t c) {
+            if (c < from) return;
+            m = c > m ? c : m;
+            const uint32_t slot = atomicAdd(&ncand, 1u);
+            if (slot < SMP_DRAW_CAND) cand[slot] = c;
+        });
+        __syncthreads();
+        return (int)ncand;
+    };
+    int n = collect((uint64_t)bound << 32);
+    if (k == 1 && n > SMP_COUNT_CAND) {     // the largest is among the threads' largest
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            const uint64_t o = __shfl_xor(m, off);
+            m = o > m ? o : m;
         }
+        if (lane == 0) tmax[tid >> 6] = m;
+        __syncthreads();
+        for (int w = 0; w < SMP_THREADS / 64; ++w) m = tmax[w] > m ? tmax[w] : m;
+        if (tid == 0) cand[0] = m;
+        __syncthreads();
+        n = 1;
+    }
+    if (n > SMP_DRAW_CAND) {
+        // Large logits beside each other, or equal ones: the k-th largest of
+        // the threads' maxima is a closer bound, reached in exactly k
+        // threads, so by at most 64 k logits.
+        tmax[tid] = m;
+        const uint64_t from = kth_largest(tmax, SMP_THREADS, k, hist, pick);
         if (tid == 0) ncand = 0;
         __syncthreads();
-        for_slices(A, list, m, tie_last, [&](uint64_t c) {
-            if (c >= prefix) cand[atomicAdd(&ncand, 1u)] = c;
-        });
+        n = collect(from);
+    }
+    if (n > SMP_COUNT_CAND) {
+        const uint64_t from = kth_largest(cand, n, k, hist, pick);
+        uint64_t own[SMP_DRAW_CAND / SMP_THREADS];
+#pragma unroll
+        for (int j = 0; j < SMP_DRAW_CAND / SMP_THREADS; ++j) {
+            const int i = tid + j * SMP_THREADS;
+            own[j] = i < n ? cand[i] : 0;
+        }
+        __syncthreads();
+        if (tid == 0) ncand = 0;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < SMP_DRAW_CAND / SMP_THREADS; ++j)
+            if (tid + j * SMP_THREADS < n && own[j] >= from) cand[atomicAdd(&ncand, 1u)] = own[j];
         __syncthreads();
         n = k;
     }
-    // rank by counting (n is a few times k), eight threads per candidate
+    // rank by counting, eight threads per candidate
     for (int i0 = 0; i0 < n; i0 += SMP_THREADS / 8) {
         const int i = i0 + (tid >> 3);
         const uint64_t mine = cand[min(i, n - 1)];
