@@ -788,8 +788,13 @@ Q4_GEMM(qm_q4_gemm_gu_bf16_big, true, true, 1, 2, 1, 8, 3, 4, true)
 // the plain f16 conversion.  One workgroup per row.  Rows of up to NV x 1024
 // values stay in registers between the sum of squares and the output, with
 // the norm weights requested beside them: one memory round trip, where
-// reading the row again cost a second (few rows: 4.8 -> 2.9 us; 4096 x 2560:
-// 15.4 -> 12.2 us).  Longer rows are read twice.
+// reading the row again cost a second.  Longer rows are read twice.  NV is 1,
+// 2 or 4 by the row's length, and lanes past its end load nothing: with four
+// loads in every lane a row of up to 1024 values took up to 1.7 times as long
+// as read twice.  Replayed graph, us, read twice / four loads / now:
+//   8192 x 64     5.6 / 9.4 / 5.4      4096 x 1280   6.2 / 7.5 / 5.8
+//   8192 x 1024  10.7 / 11.8 / 10.0    300 x 2560    2.9 / 2.6 / 2.5
+//   4096 x 2560  12.9 / 10.7 / 10.8    8192 x 4096  42.0 / 29.1 / 29.3
 template <int NV>
 __device__ __forceinline__ void rms_norm_f16_body(const RmsNormArgs& A) {
     __shared__ float red[4];
@@ -817,14 +822,14 @@ __device__ __forceinline__ void rms_norm_f16_body(const RmsNormArgs& A) {
         *reinterpret_cast<uint2*>(out + i) = make_uint2(lo, hi);
     };
     if constexpr (NV > 0) {
-        const int last = A.k - 4;                  // k % 4 == 0
         float4 v[NV];
         uint2 gw[NV];
 #pragma unroll
-        for (int j = 0; j < NV; ++j) v[j] = ld4(x + min(4 * tid + 1024 * j, last));
+        for (int j = 0; j < NV; ++j)
+            if (4 * tid + 1024 * j < A.k) v[j] = ld4(x + 4 * tid + 1024 * j);
 #pragma unroll
         for (int j = 0; j < NV; ++j)
-            gw[j] = A.norm_w ? *reinterpret_cast<const uint2*>(A.norm_w + min(4 * tid + 1024 * j, last)) : make_uint2(0, 0);
+            if (A.norm_w && 4 * tid + 1024 * j < A.k) gw[j] = *reinterpret_cast<const uint2*>(A.norm_w + 4 * tid + 1024 * j);
 #pragma unroll
         for (int j = 0; j < NV; ++j)
             if (4 * tid + 1024 * j < A.k) square(v[j]);
@@ -840,4 +845,6 @@ __device__ __forceinline__ void rms_norm_f16_body(const RmsNormArgs& A) {
     }
 }
 extern "C" __global__ __launch_bounds__(256) void qm_rms_norm_f16(RmsNormArgs A) { rms_norm_f16_body<0>(A); }
+extern "C" __global__ __launch_bounds__(256) void qm_rms_norm_f16_k1024(RmsNormArgs A) { rms_norm_f16_body<1>(A); }
+extern "C" __global__ __launch_bounds__(256) void qm_rms_norm_f16_k2048(RmsNormArgs A) { rms_norm_f16_body<2>(A); }
 extern "C" __global__ __launch_bounds__(256) void qm_rms_norm_f16_k4096(RmsNormArgs A) { rms_norm_f16_body<4>(A); }

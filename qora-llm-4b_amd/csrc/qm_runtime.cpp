@@ -55,7 +55,7 @@ struct qm_context {
     hipFunction_t f_q4_gemm[2][2][qm_q4::kNumTiles] = {};  // [x bf16][gate/up form][tile]
     hipFunction_t f_q4_gemm_big[2][2] = {};                // 64-bit lane offsets
     hipFunction_t f_rms_f16 = nullptr;
-    hipFunction_t f_rms_f16_k4096 = nullptr;  // rows of up to 4096 values
+    hipFunction_t f_rms_f16_row[3] = {};      // rows of up to 1024, 2048 and 4096 values
     hipFunction_t f_lm_head = nullptr;
     hipFunction_t f_embed = nullptr;
     hipFunction_t f_sample_pen = nullptr;
@@ -375,7 +375,9 @@ int32_t qm_create(qm_context** out, const qm_config* cfg, const char* code_objec
         if (st == QM_OK) st = load_function(c, mods[5], (stem + "big").c_str(), &c->f_q4_gemm_big[xb][gu]);
     }
     if (st == QM_OK) st = load_function(c, mods[5], "qm_rms_norm_f16", &c->f_rms_f16);
-    if (st == QM_OK) st = load_function(c, mods[5], "qm_rms_norm_f16_k4096", &c->f_rms_f16_k4096);
+    if (st == QM_OK) st = load_function(c, mods[5], "qm_rms_norm_f16_k1024", &c->f_rms_f16_row[0]);
+    if (st == QM_OK) st = load_function(c, mods[5], "qm_rms_norm_f16_k2048", &c->f_rms_f16_row[1]);
+    if (st == QM_OK) st = load_function(c, mods[5], "qm_rms_norm_f16_k4096", &c->f_rms_f16_row[2]);
     if (st == QM_OK) st = load_function(c, mods[6], "qm_q4_lm_head", &c->f_lm_head);
     if (st == QM_OK) st = load_function(c, mods[6], "qm_q4_embed", &c->f_embed);
     if (st == QM_OK) st = load_function(c, mods[7], "qm_sample_penalties", &c->f_sample_pen);
@@ -1035,8 +1037,9 @@ int32_t qm_rms_norm_f16(qm_context* c, qm_stream stream, int32_t m, int32_t k, c
     if (!all_aligned16({x, norm_w, out}))
         return fail(c, QM_ERR_INVALID_ARG, "qm_rms_norm_f16: device pointers must be 16-byte aligned");
     RmsNormArgs ra{x, norm_w, out, m, k};
-    return launch(c, k <= 4096 ? c->f_rms_f16_k4096 : c->f_rms_f16, static_cast<uint32_t>(m), 256, ra, pick(c, stream),
-                  "qm_rms_norm_f16");
+    // rows of up to 4096 values stay in registers, 1, 2 or 4 x 4 of them a thread
+    hipFunction_t f = k <= 4096 ? c->f_rms_f16_row[k <= 1024 ? 0 : k <= 2048 ? 1 : 2] : c->f_rms_f16;
+    return launch(c, f, static_cast<uint32_t>(m), 256, ra, pick(c, stream), "qm_rms_norm_f16");
 }
 
 int32_t qm_q4_lm_head(qm_context* c, qm_stream stream, int32_t vocab, int32_t hidden, const float* x,
