@@ -38,7 +38,9 @@
 // (With a v_cvt_f32_ubyteN per code, 2.4 instructions, the four launches of
 // a layer took 0.4 us more: 2560 x 12288 6.45 -> 6.31 us, 9216 x 2560 7.15
 // -> 7.02, 4096 x 2560 4.35 -> 4.26, the gate / up pair unchanged at 9.7,
-// of which 1.9 are an empty launch and 4.3 the weights at 6.2 TB/s.)
+// of which 1.9 are an empty launch and 4.3 the weights at 6.2 TB/s.)  A wave
+// whose sums say that its operands left the codes' range (q4_in_range, 0.02
+// us a launch) forms them again with the codes converted.
 // The RMSNorm is applied by linearity: y = inv_rms * (x (1 + gamma)) W, so
 // its sum of squares comes from the same x loads and the factor scales the
 // column sums.
@@ -76,6 +78,36 @@ QM_DEV void q4_accumulate(float (&acc)[16], uint2 c, float sx) {
     q4_word(acc + 8, c.y, se, so);
 }
 QM_DEV void q4_accumulate(float (&acc)[8], uint32_t c, float sx) { q4_word(acc, c, sx * QM_Q4_EVEN, sx * QM_Q4_ODD); }
+
+// Whether the wave's column sums are those of operands within the f16 codes'
+// range: one past it leaves every even column infinite or NaN, and the bits
+// lost to subnormals matter only where every sum is tiny.  Zeros are rows
+// past k.
+QM_DEV bool q4_in_range(float y, float u) {
+    constexpr uint32_t LO = 0x17800000u, INF = 0x7f800000u;   // 2^-80
+    const uint32_t a = __float_as_uint(y) & 0x7fffffffu, b = __float_as_uint(u) & 0x7fffffffu, m = a > b ? a : b;
+    if (__builtin_expect(!__any(m - LO >= INF - LO), 1)) return true;
+    return !__any(m >= INF) && (__any(m >= LO) || !__any(m));
+}
+// A lane's column partials with the codes converted to f32, for operands at
+// the ends of f32's range: the rows and their order are those of q4_tile.
+template <int T, int GROUP, int THREADS>
+QM_DEV void q4_wide_partials(float (&acc)[T], const void* codes, const uint16_t* gsc, const float* x, const uint16_t* nw,
+                             int K) {
+    const uint32_t* words = reinterpret_cast<const uint32_t*>(codes);
+#pragma unroll
+    for (int j = 0; j < T; ++j) acc[j] = 0.0f;
+#pragma unroll 1
+    for (int i = 0;; ++i) {
+        const int k = GROUP * (i / GROUP * THREADS + (int)threadIdx.x) + i % GROUP;
+        if (k >= K) break;
+        const float xn = nw ? x[k] * (1.0f + f16_to_f32(nw[k])) : x[k];
+        const float sx = f16_to_f32(gsc[k]) * xn;
+#pragma unroll
+        for (int j = 0; j < T; ++j)
+            acc[j] = fmaf((float)((words[(size_t)k * (T / 8) + j / 8] >> (4 * (j % 8))) & 15u), sx, acc[j]);
+    }
+}
 
 // Wave-level sum of each of a lane's T column partials by transpose-reduce:
 // each step pairs lane l with l ^ 32, ^16, ^8 (and ^4 for T = 16), and each
@@ -261,7 +293,7 @@ QM_DEV void q4_tile(const Q4GemvArgs& A, int p, int tile, float (*red)[33]) {
     const int lane = tid & 63, wv = tid >> 6;
 #pragma unroll
     for (int j = 0; j < T; ++j) acc[j] = fmaf(QM_Q4_SUM, acc[j], -8.0f * bsum);
-    const float cs = q4_wave_reduce<T>(acc, lane);
+    float cs = q4_wave_reduce<T>(acc, lane);
     float cs_u = 0.0f;
     if (GATE_UP) {
 #pragma unroll
@@ -269,6 +301,17 @@ QM_DEV void q4_tile(const Q4GemvArgs& A, int p, int tile, float (*red)[33]) {
         cs_u = q4_wave_reduce<T>(reinterpret_cast<float(&)[T]>(acc_u), lane);
     }
     const float ssw = NORM ? wave_sum64(ss) : 0.0f;
+    if (!q4_in_range(cs, cs_u)) {
+        auto wide = [&](const CodeT* c, const uint16_t* sc, float b) {
+            float w[T];
+            q4_wide_partials<T, PAIR ? 2 : 1, THREADS>(w, c, sc, A.x, NORM ? nwp : nullptr, K);
+#pragma unroll
+            for (int j = 0; j < T; ++j) w[j] = fmaf(-8.0f, b, w[j]);
+            return q4_wave_reduce<T>(w, lane);
+        };
+        cs = wide(codes, gsc, bsum);
+        if (GATE_UP) cs_u = wide(codes_u, gsc_u, bsum_u);
+    }
     if ((lane & (64 / T - 1)) == 0) {
         red[wv][q4_col<T>(lane)] = cs;
         if (GATE_UP) red[wv][16 + q4_col<T>(lane)] = cs_u;

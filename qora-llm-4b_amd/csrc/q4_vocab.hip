@@ -27,8 +27,8 @@
 #include "qm_kernel_args.h"
 
 // 8 codes (one 32-bit word: columns 8t .. 8t + 7 of a group) against the
-// matching x values (scaled by QM_Q4_EVEN / QM_Q4_ODD); returns the sum of
-// q * x over them / QM_Q4_SUM.
+// matching x values, scaled for the codes' f16 form; returns the sum of q * x
+// over them, / the sum's factor.
 QM_DEV float q4_word_dot(uint32_t w, const float* xw, float acc) {
     q4_half2 h[4];
     q4_halves(w, h);
@@ -97,10 +97,16 @@ extern "C" __global__ __launch_bounds__(1024) void qm_q4_lm_head(LmHeadArgs A) {
 #pragma unroll
     for (int e = 0; e < 32; ++e) sx += xs[e];
     sx *= 8.0f;
+    float mag = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 32; ++e) mag = fmaxf(mag, fabsf(xs[e]));
+    // (moved by 2^24 where they come near an end of f32's range)
+    const float range = mag >= 0x1p115f ? 0x1p-24f : mag > 0.0f && mag < 0x1p-88f ? 0x1p24f : 1.0f;
+    const float qsum = QM_Q4_SUM / range;
 #pragma unroll
     for (int e = 0; e < 32; e += 2) {
-        xs[e] *= QM_Q4_EVEN;
-        xs[e + 1] *= QM_Q4_ODD;
+        xs[e] *= QM_Q4_EVEN * range;
+        xs[e + 1] *= QM_Q4_ODD * range;
     }
 
     const int nsb = (A.vocab + 4 * LMH_SB - 1) / (4 * LMH_SB);
@@ -122,7 +128,7 @@ extern "C" __global__ __launch_bounds__(1024) void qm_q4_lm_head(LmHeadArgs A) {
             d = q4_word_dot(c[b].y, &xs[8], d);
             d = q4_word_dot(c[b].z, &xs[16], d);
             d = q4_word_dot(c[b].w, &xs[24], d);
-            const float p = row_sum16(f16_to_f32(sc[b]) * fmaf(d, QM_Q4_SUM, -sx));
+            const float p = row_sum16(f16_to_f32(sc[b]) * fmaf(d, qsum, -sx));
             if (sl == 0) part[b][seg] = p;
         }
         __syncthreads();

@@ -77,8 +77,10 @@ QM_DEV float bf16_to_f32(uint16_t h) { return __builtin_bit_cast(float, (uint32_
 // 19 with a v_cvt_f32_ubyteN per code).  The factors go into the f32 side:
 // the operand of an even column times QM_Q4_EVEN, of an odd one times
 // QM_Q4_ODD, and the sum times QM_Q4_SUM, all powers of two, so the results
-// are the same bits as with the codes converted (half of the 2^24 is put on
-// each side of the sum, so that neither end of f32's range comes near).
+// are the same bits as with the codes converted, as long as no operand times
+// QM_Q4_EVEN overflows (from 2^116) and no product / QM_Q4_SUM is subnormal
+// (operands below 2^-114; half of the 2^24 is put on each side of the sum).
+// Kernels that take operands as they come look for those and do without.
 #define QM_Q4_EVEN 4096.0f
 #define QM_Q4_ODD 256.0f
 #define QM_Q4_SUM 4096.0f

@@ -77,6 +77,54 @@ def test_q4_gemv_range(ctx, k, n, power):
     assert np.array_equal(scaled, np.ldexp(got, power))
 
 
+def _few_large(x, packed, scales, rng):
+    """12 rows of x, and the power of two that takes x and every column's sum
+    of 16 |scale x| just under f32's end (so that x (q - 8) sums stay finite)."""
+    x = np.where(np.isin(np.arange(len(x)), rng.choice(len(x), 12, replace=False)), x, 0).astype(np.float32)
+    top = 16.0 * (np.abs(x).astype(np.float64) @ np.abs(W.f16_value(scales)).astype(np.float64)).max()
+    return x, 127 - int(np.ceil(np.log2(max(top, np.abs(x).max()))))
+
+
+@pytest.mark.parametrize("k,n", [(37, 64), (2560, 4096), (2560, 2560), (3001, 4096), (4096, 32), (9216, 2560)])
+def test_q4_gemv_range_ends(ctx, k, n):
+    """Up to the ends of f32's range x times a power of two gives y times it,
+    bit for bit: |scale x| past 2^116, where the f16 codes' factor would
+    overflow, and down to 2^-125, where q scale x over the sum's factor would
+    be subnormal (row pairs and single rows, tiles of 8 and 16 columns, each
+    kernel form)."""
+    rng = np.random.default_rng(k + n)
+    w = W.q4_gemv_workload(k, n, seed=k + n)
+    w["scales"] = W.f16_bits(np.maximum(W.f16_value(w["scales"]), 0.002))
+    x, power = _few_large(w["x"], w["packed"], w["scales"], rng)
+    sx = np.abs(x).max() * W.f16_value(w["scales"]).max()
+    print(f"case: q4 gemv k={k} n={n}, x * 2^{power}", flush=True)
+    assert np.ldexp(sx, power) > 2.0 ** 117
+    got = run_gpu(ctx, x, w["packed"], w["scales"])
+    assert np.array_equal(run_gpu(ctx, np.ldexp(x, power), w["packed"], w["scales"]), np.ldexp(got, power))
+    # 12-bit x, so that scale x is exact in the sums that take it unrounded too
+    x = (rng.choice([-1.0, 1.0], k) * (1.0 + rng.integers(0, 2048, k) / 2048.0)).astype(np.float32)
+    power = -125 - int(np.floor(np.log2(W.f16_value(w["scales"]).min())))
+    print(f"case: q4 gemv k={k} n={n}, x * 2^{power}", flush=True)
+    got = run_gpu(ctx, x, w["packed"], w["scales"])
+    assert np.array_equal(run_gpu(ctx, np.ldexp(x, power), w["packed"], w["scales"]), np.ldexp(got, power))
+
+
+@pytest.mark.parametrize("k,n", [(37, 64), (2560, 4128)])
+@pytest.mark.parametrize("zero", ["gate", "up"])
+def test_q4_gate_up_range_end(ctx, zero, k, n):
+    """|scale x| past 2^116 on one side and zero scales on the other: the sums
+    are finite, silu(g) is 0, -0 or g, and the product is zero."""
+    rng = np.random.default_rng(k + n)
+    packed, scales = W.q4_random_weight(k, n, rng)
+    x, power = _few_large(rng.standard_normal(k).astype(np.float32), packed, scales, rng)
+    nil = np.zeros_like(scales)
+    gate, up = repack(ctx, packed, nil if zero == "gate" else scales), repack(ctx, packed, nil if zero == "up" else scales)
+    out = ctx.upload(np.full(n, np.nan, np.float32))
+    print(f"case: q4 gate/up k={k} n={n}, zero {zero}, x * 2^{power}", flush=True)
+    ctx.q4_gate_up(k, n, ctx.upload(np.ldexp(x, power)), None, *gate, *up, out)
+    assert np.array_equal(ctx.download(out, (n,), np.float32), np.zeros(n, np.float32))
+
+
 def test_q4_gemv_multi_layer_projections(ctx):
     """in_proj_qkv, in_proj_z, in_proj_a, in_proj_b of one input in one launch,
     each output as its own qm_q4_gemv would give it (bit for bit) and within

@@ -80,6 +80,22 @@ def test_lm_head_rows_per_workgroup_and_range(ctx, vocab, hidden, power):
     assert np.array_equal(_lm_head(ctx, np.ldexp(x, power), None, packed, scales), np.ldexp(got, power))
 
 
+@pytest.mark.parametrize("vocab,hidden", [(33, 512), (1000, 2560), (257, 8192)])
+def test_lm_head_range_ends(ctx, vocab, hidden):
+    """Up to the ends of f32's range x times a power of two gives the logits
+    times it, bit for bit: |x| past 2^116, where the f16 codes' factor would
+    overflow, and down to 2^-125, where q x over the sum's factor would be
+    subnormal."""
+    rng, packed, scales = _embed(vocab, hidden, vocab)
+    x = np.where(np.isin(np.arange(hidden), rng.choice(hidden, 5, replace=False)), 1.0 + rng.random(hidden), 0.0)
+    for x, scales, power in ((x.astype(np.float32), scales, 119),
+                             ((1.0 + rng.random(hidden)).astype(np.float32),
+                              W.f16_bits(np.maximum(W.f16_value(scales), 0.002) * 8192.0), -125)):
+        print(f"case: lm_head {vocab} x {hidden}, x * 2^{power}", flush=True)
+        got = _lm_head(ctx, x, None, packed, scales)
+        assert np.array_equal(_lm_head(ctx, np.ldexp(x, power), None, packed, scales), np.ldexp(got, power))
+
+
 def test_embed_rows_exact(ctx):
     vocab, hidden = 248320, 2560
     _, packed, scales = _embed(vocab, hidden, 82)
