@@ -97,12 +97,15 @@ extern "C" __global__ __launch_bounds__(1024) void qm_q4_lm_head(LmHeadArgs A) {
 #pragma unroll
     for (int e = 0; e < 32; ++e) sx += xs[e];
     sx *= 8.0f;
-    float mag = 0.0f;
+    // the largest |x| moves the factors by 2^24 where it comes near an end of
+    // f32's range
+    float top[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int e = 0; e < 32; ++e) mag = fmaxf(mag, fabsf(xs[e]));
-    // (moved by 2^24 where they come near an end of f32's range)
-    const float range = mag >= 0x1p115f ? 0x1p-24f : mag > 0.0f && mag < 0x1p-88f ? 0x1p24f : 1.0f;
-    const float qsum = QM_Q4_SUM / range;
+    for (int e = 0; e < 32; ++e) top[e & 3] = fmaxf(top[e & 3], fabsf(xs[e]));
+    const float mag = fmaxf(fmaxf(top[0], top[1]), fmaxf(top[2], top[3]));
+    const bool high = mag >= 0x1p115f, low = mag > 0.0f && mag < 0x1p-88f;
+    const float range = high ? 0x1p-24f : low ? 0x1p24f : 1.0f;
+    const float qsum = high ? QM_Q4_SUM * 0x1p24f : low ? QM_Q4_SUM * 0x1p-24f : QM_Q4_SUM;
 #pragma unroll
     for (int e = 0; e < 32; e += 2) {
         xs[e] *= QM_Q4_EVEN * range;
