@@ -113,8 +113,9 @@ enum {
     QM_OPT_DN_DECODE_THREADS = 1,  /* threads per v-head workgroup: 256, 512, 1024 */
     QM_OPT_GQA_DECODE_CHUNK = 2,   /* keys per split-K workgroup (mult. 64)*/
     QM_OPT_GQA_PREFILL_ORDER = 3   /* row-block order of the causal prefill:
-                                      1 longest first, 2 packed; results are
-                                      bit-identical */
+                                      1 longest first, 2 packed (which also
+                                      takes 48-row blocks at every length);
+                                      results are bit-identical */
 };
 int32_t     qm_set_option(qm_context* ctx, int32_t option, int64_t value);
 

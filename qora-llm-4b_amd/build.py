@@ -101,6 +101,13 @@ def build_plan_test() -> None:
           str(ROOT / "tests" / "cpp" / "gqa_plan_test.cpp"), "-o", str(LIB / "gqa_plan_test")])
 
 
+def build_dispatch_test() -> None:
+    """tests/cpp/dispatch_test.cpp: the host's choices of kernel on the CPU
+    (g++ only, no device code; test infrastructure)."""
+    _run(["g++", "-O2", "-std=c++17", "-Wall", "-Wextra", "-I", str(CSRC),
+          str(ROOT / "tests" / "cpp" / "dispatch_test.cpp"), "-o", str(LIB / "dispatch_test")])
+
+
 if __name__ == "__main__":
     build()
     if "--no-oracle" not in sys.argv:
@@ -108,4 +115,5 @@ if __name__ == "__main__":
         build_host_test()
         build_file_test()
         build_plan_test()
+        build_dispatch_test()
     print("built:", ", ".join(sorted(p.name for p in LIB.iterdir())))

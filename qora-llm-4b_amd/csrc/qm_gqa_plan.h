@@ -10,6 +10,19 @@
 #include "qm_kernel_args.h"
 
 namespace qm_plan {
+// 16-row groups per row block of the attention: blocks of 32 rows (8 waves)
+// where blocks of 48 (12 waves) leave CUs idle or the longest block's chain of
+// tiles bounds the call; above, a tile's fetch feeding twelve waves is worth
+// more.  Both reasons lie in the number of blocks a CU gets, so the line is
+// drawn in tokens per CU, where it was measured on 256, us, 32 / 48: 300
+// tokens 25.2 / 30.6, 700 34.8 / 42.7, 2048 70.3 / 83.4, 3000 101 / 123, 4200
+// 169 / 178, 4400 183 / 187, 4600 198 / 196, 5000 235 / 225 (blocks of 16:
+// 27.7, 42.8, 107, 208).  A forced packed order (mode 2) is a plan of 48-row
+// blocks.
+inline int32_t gqp_row_groups(int32_t S, int32_t num_cu, int64_t mode) {
+    return 256 * static_cast<int64_t>(S) <= 4400 * static_cast<int64_t>(num_cu) && mode != 2 ? 2 : 3;
+}
+
 // Row-block order of the attention's per-group queues.  Each kv group's
 // blocks go to whichever of its `bins` workgroups draws next, so the order
 // decides how the causal triangle's unequal blocks pack.  Block tb (rows

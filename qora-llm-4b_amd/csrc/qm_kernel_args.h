@@ -139,8 +139,9 @@ struct GqaPrefillArgs {
 };
 
 // The attention kernel's arguments: the shared ones plus the order in which
-// each kv group's queue hands out its 48-row blocks (block 0 = rows 0..47).
-// ordered = 0: the n-th draw is the n-th longest block (nblk - 1 - n).
+// each kv group's queue hands out its row blocks (block 0 = the first rows).
+// ordered = 0: the n-th draw is the n-th longest block (nblk - 1 - n), as
+// always with 32-row blocks; an order is one of 48-row blocks.
 #define QM_GQA_PREFILL_ORDER_MAX 1024
 struct GqaPrefillAttnArgs {
     GqaPrefillArgs a;

@@ -867,14 +867,7 @@ int32_t qm_gqa_prefill(qm_context* c, qm_stream stream, int32_t seq_len, const u
     st = launch(c, c->f_gqp_kv, static_cast<uint32_t>(s_pad / 64) * QM_GQA_KV_HEADS, c->gqp_kv_threads, ga, s,
                 "qm_gqa_prefill_kv");
     if (st != QM_OK) return st;
-    // Row blocks of 32 rows (8 waves) up to 4400 tokens, where blocks of 48
-    // (12 waves) leave CUs idle or the longest block's chain of tiles bounds
-    // the call; above, a tile's fetch feeding twelve waves is worth more.
-    // Measured, us, 32 / 48: 300 tokens 25.2 / 30.6, 700 34.8 / 42.7, 2048
-    // 70.3 / 83.4, 3000 101 / 123, 4200 169 / 178, 4400 183 / 187, 4600
-    // 198 / 196, 5000 235 / 225 (blocks of 16: 27.7, 42.8, 107, 208).  A
-    // forced packed order is a plan of 48-row blocks.
-    const int32_t groups = seq_len <= 4400 && c->opt_gqp_order != 2 ? 2 : 3;
+    const int32_t groups = qm_plan::gqp_row_groups(seq_len, c->num_cu, c->opt_gqp_order);
     // persistent: one workgroup per CU (a multiple of the 4 kv groups), no
     // more than there are row blocks
     const int32_t nblk = (seq_len + 16 * groups - 1) / (16 * groups);
