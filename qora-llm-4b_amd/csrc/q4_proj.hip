@@ -815,11 +815,15 @@ __device__ __forceinline__ void q4_gemm_body(const Q4GemmArgs& A) {
     Q4_GEMM(qm_q4_gemm_bf16_m##MI##n##NJ##w##WN##k##WK, true, false, MI, NJ, WN, WK, NST, OCC)
 #define Q4_GEMM_GATE_UP(MI, NJ, WN, WK, NST, OCC, ...)                                             \
     Q4_GEMM(qm_q4_gemm_gu_f16_m##MI##n##NJ##w##WN##k##WK, false, true, MI, NJ, WN, WK, NST, OCC)   \
+    Q4_GEMM_GATE_UP_BF16(MI, NJ, WN, WK, NST, OCC)
+#define Q4_GEMM_GATE_UP_BF16(MI, NJ, WN, WK, NST, OCC, ...)                                        \
     Q4_GEMM(qm_q4_gemm_gu_bf16_m##MI##n##NJ##w##WN##k##WK, true, true, MI, NJ, WN, WK, NST, OCC)
 QM_Q4_TILES_ONE_WAVE(Q4_GEMM_PLAIN)
+QM_Q4_TILES_GATE_UP_BF16(Q4_GEMM_PLAIN)
 QM_Q4_TILES_PAIRED(Q4_GEMM_PLAIN)
 QM_Q4_TILES_ODD(Q4_GEMM_PLAIN)
 QM_Q4_TILES_ONE_WAVE(Q4_GEMM_GATE_UP)
+QM_Q4_TILES_GATE_UP_BF16(Q4_GEMM_GATE_UP_BF16)
 QM_Q4_TILES_PAIRED(Q4_GEMM_GATE_UP)
 Q4_GEMM(qm_q4_gemm_f16_big, false, false, 1, 2, 1, 8, 3, 4, true)
 Q4_GEMM(qm_q4_gemm_bf16_big, true, false, 1, 2, 1, 8, 3, 4, true)

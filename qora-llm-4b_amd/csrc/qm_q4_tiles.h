@@ -27,7 +27,9 @@
     X(3, 4, 1, 8, 2, 2, 1058, 1370, 1285, 1426) \
     X(4, 2, 1, 8, 2, 2, 792, 1105, 896, 1031)   \
     X(5, 4, 1, 4, 2, 1, 932, 1050, 1008, 1068)  \
-    X(6, 4, 1, 4, 2, 1, 1075, 1210, 1097, 1170) \
+    X(6, 4, 1, 4, 2, 1, 1075, 1210, 1097, 1170)
+// no call takes its gate/up form with an f16 x: not built
+#define QM_Q4_TILES_GATE_UP_BF16(X)             \
     X(8, 4, 1, 4, 2, 1, 1348, 1463, 1364, 1442)
 #define QM_Q4_TILES_PAIRED(X)                   \
     X(3, 2, 2, 4, 2, 4, 641, 627, 797, 669)     \
@@ -51,18 +53,25 @@ namespace qm_q4 {
 struct Tile {
     const char* name;            // kernel name suffix
     int32_t mi, nj, wn, wk;
+    int32_t gate_up;             // gate/up forms: 1 for an f16 x, 2 for a bf16 one
     int32_t alone[2], shared[2]; // [x is bf16]
 };
 
-#define QM_Q4_TILE_ROW(MI, NJ, WN, WK, NST, OCC, AF, SF, AB, SB) \
-    {"m" #MI "n" #NJ "w" #WN "k" #WK, MI, NJ, WN, WK, {AF, AB}, {SF, SB}},
-constexpr Tile kTiles[] = {QM_Q4_TILES_ONE_WAVE(QM_Q4_TILE_ROW) QM_Q4_TILES_PAIRED(QM_Q4_TILE_ROW)
-                           QM_Q4_TILES_ODD(QM_Q4_TILE_ROW)};
+#define QM_Q4_TILE_ROW(GU, MI, NJ, WN, WK, AF, SF, AB, SB) \
+    {"m" #MI "n" #NJ "w" #WN "k" #WK, MI, NJ, WN, WK, GU, {AF, AB}, {SF, SB}},
+#define QM_Q4_ROW_GATE_UP(MI, NJ, WN, WK, NST, OCC, ...) QM_Q4_TILE_ROW(3, MI, NJ, WN, WK, __VA_ARGS__)
+#define QM_Q4_ROW_GATE_UP_BF16(MI, NJ, WN, WK, NST, OCC, ...) QM_Q4_TILE_ROW(2, MI, NJ, WN, WK, __VA_ARGS__)
+#define QM_Q4_ROW_PLAIN(MI, NJ, WN, WK, NST, OCC, ...) QM_Q4_TILE_ROW(0, MI, NJ, WN, WK, __VA_ARGS__)
+constexpr Tile kTiles[] = {QM_Q4_TILES_ONE_WAVE(QM_Q4_ROW_GATE_UP) QM_Q4_TILES_GATE_UP_BF16(QM_Q4_ROW_GATE_UP_BF16)
+                           QM_Q4_TILES_PAIRED(QM_Q4_ROW_GATE_UP) QM_Q4_TILES_ODD(QM_Q4_ROW_PLAIN)};
+#undef QM_Q4_ROW_PLAIN
+#undef QM_Q4_ROW_GATE_UP_BF16
+#undef QM_Q4_ROW_GATE_UP
 #undef QM_Q4_TILE_ROW
 constexpr int kBigTile = 0;      // the tile of the form with 64-bit lane offsets
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 
-inline bool has_gate_up(const Tile& t) { return (t.wn == 1 ? t.wk : t.wn) % 2 == 0; }
+inline bool has_gate_up(const Tile& t, bool bf16) { return t.gate_up >> bf16 & 1; }
 
 inline int64_t tile_grid(const Tile& t, int64_t m, int64_t n, bool gate_up) {
     const int64_t rows = 16 * t.mi, cols = 16 * t.nj * (gate_up && t.wn > 1 ? t.wn / 2 : t.wn);
@@ -75,13 +84,17 @@ inline int64_t tile_grid(const Tile& t, int64_t m, int64_t n, bool gate_up) {
 // loads less per product, a small one, or one that splits k over its waves,
 // fills the CUs and shortens the chain of stages when there are few rows.
 // Over the measured sizes the choice was within 1% of the best of these tiles
-// on average (20% at worst).
+// on average (20% at worst).  From k = 512 on no size of a sweep over 14
+// weight shapes and 1 to 8192 rows took longer than with the dequantize-to-LDS
+// form these tiles replace; below, where a call is little more than its launch
+// and epilogue, the best of them take 0.1 to 0.9 us more than that form did at
+// some sizes (1200 x 32 x 2560 5.3 -> 6.1 us, 1 x 128 x 32 1.8 -> 2.3).
 inline int pick_tile(int64_t m, int64_t k, int64_t n, bool bf16, bool gate_up, int num_cu) {
     int best = -1;
     int64_t best_ns = 0;
     for (int i = 0; i < kNumTiles; ++i) {
         const Tile& t = kTiles[i];
-        if (gate_up && !has_gate_up(t)) continue;
+        if (gate_up && !has_gate_up(t, bf16)) continue;
         const int64_t groups = gate_up && t.wn == 1 ? t.wk / 2 : t.wk;
         const int64_t stages = ((k / 32 + 1) / 2 + groups - 1) / groups;
         const int64_t per_cu = (tile_grid(t, m, n, gate_up) + num_cu - 1) / num_cu;

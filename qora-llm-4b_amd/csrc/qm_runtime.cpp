@@ -370,7 +370,7 @@ int32_t qm_create(qm_context** out, const qm_config* cfg, const char* code_objec
         const int xb = i & 1, gu = i >> 1;
         const std::string stem = std::string("qm_q4_gemm_") + (gu ? "gu_" : "") + (xb ? "bf16_" : "f16_");
         for (int t = 0; t < qm_q4::kNumTiles && st == QM_OK; ++t)
-            if (!gu || qm_q4::has_gate_up(qm_q4::kTiles[t]))
+            if (!gu || qm_q4::has_gate_up(qm_q4::kTiles[t], xb))
                 st = load_function(c, mods[5], (stem + qm_q4::kTiles[t].name).c_str(), &c->f_q4_gemm[xb][gu][t]);
         if (st == QM_OK) st = load_function(c, mods[5], (stem + "big").c_str(), &c->f_q4_gemm_big[xb][gu]);
     }

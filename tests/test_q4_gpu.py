@@ -417,8 +417,8 @@ def _w_bf16(packed, scales):
 def test_q4_gemm_bf16_input(ctx, name, m):
     """out_proj on a mixer prefill output (bf16 [T][4096]) with the residual
     added in place (gemv.rs:1222-1223), and bf16 inputs on the other tile
-    shapes (in_proj_qkv 128 x 256, down_proj 128 x 128, the 32-wide
-    in_proj_a 16 x 32).  Against the oracle on the bf16
+    shapes (a wide and a narrow output, and the 32-wide in_proj_a).
+    Against the oracle on the bf16
     values: |y - y_ref| <= (2^-8 + 2^-11 + 1e-4) sum_k |x_k W_kj|.  Against
     the arithmetic the kernel states (x times bf16(f16(s (q - 8))) summed in
     fp32): within 1e-5 of max |y|, where a W rounded only to f16 would differ
@@ -453,8 +453,8 @@ def test_q4_gemm_gate_up(ctx, n, m, x_dtype):
     """The prefill MLP's gate/up GEMMs and silu(g) * u (gemv.rs:1231-1237)
     in one launch, written as bf16.  Bar: the GEMM bar carried through
     silu(g) * u, plus the bf16 rounding of the output.  n = 2592 ends in a
-    partial 128-column tile of the 8-column device layout; m = 1000 on
-    n = 9216 runs 576 workgroups, several per CU."""
+    partial workgroup tile of the 8-column device layout; m = 1000 on
+    n = 9216 runs several workgroups per CU."""
     k = 2560
     rng = np.random.default_rng(n + m)
     (gp, gs), (up, us) = W.q4_random_weight(k, n, rng), W.q4_random_weight(k, n, rng)
@@ -622,6 +622,67 @@ def test_q4_gemm_tiles(ctx, tile, m, k, n, x_dtype):
     err = np.abs(got - ref) / (bound + 1e-30)
     print(f"max|d|/bound {err.max():.3e}")
     assert np.all(err <= 1.0)
+
+
+# The remaining tiles of each form, operand type and device layout (those that
+# a call can take at all), and the MLP's gate/up of short prompts.
+GEMM_TILES_BY_TYPE = [
+    ("m1n4w1k8", "f16", 1, 288, 8224), ("m1n4w1k8", "bf16", 1, 288, 8224), ("m1n4w1k8", "f16", 257, 96, 928),
+    ("m2n4w1k8", "f16", 514, 288, 928), ("m2n4w1k8", "bf16", 514, 288, 928), ("m4n2w1k8", "bf16", 49, 288, 4128),
+    ("m8n4w1k4", "f16", 337, 160, 4128), ("m8n4w1k4", "f16", 3505, 160, 416), ("m8n4w1k4", "bf16", 3266, 96, 544),
+    ("m8n4w4k1", "f16", 3457, 160, 1568), ("m8n4w4k1", "bf16", 3457, 160, 1568),
+    ("m8n4w4k2", "f16", 3458, 96, 1568), ("m8n4w4k2", "bf16", 3458, 96, 1568),
+    ("gate/up m1n4w1k8", "f16", 1, 160, 8224), ("gate/up m1n4w1k8", "bf16", 1, 160, 8224),
+    ("gate/up m1n4w1k8", "f16", 257, 96, 928), ("gate/up m1n4w1k8", "f16", 5, 2560, 9216),
+    ("gate/up m2n4w1k8", "f16", 514, 160, 928), ("gate/up m2n4w1k8", "bf16", 514, 160, 928),
+    ("gate/up m3n2w2k4", "f16", 289, 160, 4128), ("gate/up m3n2w2k4", "bf16", 289, 160, 4128),
+    ("gate/up m3n2w2k4", "f16", 3073, 160, 224), ("gate/up m3n2w2k4", "bf16", 3073, 160, 224),
+    ("gate/up m3n2w2k4", "f16", 100, 2560, 9216), ("gate/up m3n2w2k4", "f16", 130, 2560, 9216),
+    ("gate/up m4n2w1k8", "bf16", 49, 160, 4128), ("gate/up m8n4w1k4", "bf16", 289, 96, 4128),
+    ("gate/up m8n4w1k4", "bf16", 3457, 96, 416)]
+
+
+@pytest.mark.parametrize("tile,x_dtype,m,k,n", GEMM_TILES_BY_TYPE)
+def test_q4_gemm_tiles_by_type(ctx, tile, x_dtype, m, k, n):
+    """As test_q4_gemm_tiles, at sizes that take the tile for one operand type."""
+    test_q4_gemm_tiles(ctx, tile, m, k, n, x_dtype)
+
+
+@pytest.mark.parametrize("gate_up", [False, True])
+@pytest.mark.parametrize("x_dtype", ["f16", "bf16"])
+def test_q4_gemm_long_k_forms(ctx, x_dtype, gate_up):
+    """The forms with 64-bit lane offsets, x zero but in some rows of k, both
+    ends and both sides of 2^22 and 2^23 among them: sums of 64 products
+    (fp32, at most 72 2^-24 of sum |x w| in any order; gate/up as above), so
+    that a row dropped, repeated or taken from elsewhere shows."""
+    m, k, n = 2, (1 << 23) + 32, 32
+    rng = np.random.default_rng(29 + gate_up)
+    rows = np.unique(np.concatenate([[0, 31, 32, 63, 64, (1 << 22) - 1, 1 << 22, (1 << 23) - 1, 1 << 23, k - 1],
+                                     rng.integers(0, k, 54)]))
+    x = np.zeros((m, k), np.float32)
+    x[:, rows] = rng.standard_normal((m, len(rows)))
+    bits = W.bf16_bits(x) if x_dtype == "bf16" else W.f16_bits(x)
+    xv = (W.bf16_value(bits[:, rows]) if x_dtype == "bf16" else W.f16_value(bits[:, rows])).astype(np.float64)
+    pairs = [W.q4_random_weight(k, n, rng) for _ in range(1 + gate_up)]
+    ws = [(p[rows], s[rows]) for p, s in pairs]
+    ws = [(_w_bf16(*p) if x_dtype == "bf16" else W.f16_value(W.f16_bits(W.q4_dequant(*p)))).astype(np.float64)
+          for p in ws]
+    sums, mags = [xv @ w for w in ws], [72 * 2.0 ** -24 * (np.abs(xv) @ np.abs(w)) for w in ws]
+    dev = [repack(ctx, *p) for p in pairs]
+    dt = M.QM_BF16 if x_dtype == "bf16" else M.QM_F16
+    print(f"case: q4 gemm long k, {x_dtype}{' gate/up' if gate_up else ''}", flush=True)
+    if gate_up:
+        y = ctx.upload(np.full((m, n), 0x7fc0, np.uint16))
+        ctx.q4_gemm_gate_up(m, k, n, ctx.upload(bits), *dev[0], *dev[1], y, x_dtype=dt)
+        got = W.bf16_value(ctx.download(y, (m, n), np.uint16)).astype(np.float64)
+        silu = sums[0] / (1.0 + np.exp(-sums[0]))
+        ref = silu * sums[1]
+        bound = 1.1 * mags[0] * np.abs(sums[1]) + np.abs(silu) * mags[1] + (2.0 ** -8 + 1e-6) * np.abs(ref)
+    else:
+        y = ctx.upload(np.full((m, n), np.nan, np.float32))
+        ctx.q4_gemm(m, k, n, ctx.upload(bits), *dev[0], y=y, x_dtype=dt)
+        got, ref, bound = ctx.download(y, (m, n), np.float32).astype(np.float64), sums[0], mags[0]
+    assert np.all(np.abs(got - ref) <= bound + 1e-30)
 
 
 def test_q4_gemm_long_k(ctx):
