@@ -301,6 +301,14 @@ QM_DEV void q4_tile(const Q4GemvArgs& A, int p, int tile, float (*red)[33]) {
         cs_u = q4_wave_reduce<T>(reinterpret_cast<float(&)[T]>(acc_u), lane);
     }
     const float ssw = NORM ? wave_sum64(ss) : 0.0f;
+    auto publish = [&] {
+        if ((lane & (64 / T - 1)) == 0) {
+            red[wv][q4_col<T>(lane)] = cs;
+            if (GATE_UP) red[wv][16 + q4_col<T>(lane)] = cs_u;
+        }
+    };
+    publish();
+    if (lane == 0) red[wv][32] = ssw;
     if (!q4_in_range(cs, cs_u)) {
         auto wide = [&](const CodeT* c, const uint16_t* sc, float b) {
             float w[T];
@@ -311,12 +319,8 @@ QM_DEV void q4_tile(const Q4GemvArgs& A, int p, int tile, float (*red)[33]) {
         };
         cs = wide(codes, gsc, bsum);
         if (GATE_UP) cs_u = wide(codes_u, gsc_u, bsum_u);
+        publish();
     }
-    if ((lane & (64 / T - 1)) == 0) {
-        red[wv][q4_col<T>(lane)] = cs;
-        if (GATE_UP) red[wv][16 + q4_col<T>(lane)] = cs_u;
-    }
-    if (lane == 0) red[wv][32] = ssw;
     __syncthreads();
     float y = 0.0f, u = 0.0f, sst = 0.0f;
     if (tid < T) {
