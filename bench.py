@@ -962,7 +962,7 @@ def run_sample(args, ctx):
     nbytes = V * 4 * 2 + SAMPLE_GEN * 4       # logits read by the penalty pass and the selection
     return {
         "tokens": K, "total_ms": t0.elapsed_ms(t1), "wall_s": wall,
-        "dominant": "qm_sample (penalties + select + merge/draw, 3 launches)",
+        "dominant": "qm_sample (penalties and slice maxima, then select and draw, 2 launches)",
         "roofline": {"bound": "hbm", "achieved": nbytes / (ms * 1e-3), "peak": HBM_PEAK,
                      "kernel_ms": ms, "bytes_per_launch": nbytes},
         "config": {"workload": "next-token sampling over 248320 logits: presence penalty (1000 ids), top_k 20, "

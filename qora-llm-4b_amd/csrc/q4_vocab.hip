@@ -45,7 +45,7 @@ QM_DEV float q4_word_dot(uint32_t w, const float* xw, float acc) {
 // one row of the batch: its partial sum goes to LDS, and after LMH_SB
 // batches one thread per row adds the row's G / 16 partials in a fixed
 // order.  Workgroups stride over these super-batches of 4 LMH_SB rows.
-// 248,320 x 2560: 64.5 us (5.5 TB/s); 73.6 with a conversion per code and
+// 248,320 x 2560: 64-67 us (5.4-5.6 TB/s); 72-75 with a conversion per code and
 // four workgroups per CU.  Loading the next super-batch while this one is
 // summed changed it by less than the runs differ.
 #define LMH_SB 8

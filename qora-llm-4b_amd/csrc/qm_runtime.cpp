@@ -1053,9 +1053,10 @@ int32_t qm_q4_lm_head(qm_context* c, qm_stream stream, int32_t vocab, int32_t hi
         c->lm_head_wg_per_cu = n;
     }
     // super-batches of 32 rows over up to 16 waves per CU, as many workgroups on every CU.  At hidden 2560 (five
-    // waves a workgroup) 3 per CU take 62 us for 248,320 rows, 4 per CU 69 (they compete for the same stream) and a
+    // waves a workgroup) 3 per CU take 62-65 us for 248,320 rows, 4 per CU 69 (they compete for the same stream) and a
     // grid rounded down until every workgroup has the same count 69 / 72: some CUs then have one fewer.  At hidden
-    // 512, 1024 and 4096 16 waves are within 2% of the best.
+    // 512, 1024 and 4096 16 waves are within 2% of the best; above, one workgroup per CU (4608, 5120, 6144, 8192) takes
+    // 0.84 to 1.02 of the time of as many as fit, over 1000 to 151,936 rows.
     const int64_t nsb = (static_cast<int64_t>(vocab) + 31) / 32;
     const int64_t wgs = std::min<int64_t>(c->lm_head_wg_per_cu, std::max(1, 16 * 64 / block));
     const int64_t grid = std::min(nsb, c->num_cu * wgs);

@@ -41,7 +41,7 @@
 // What bounded the longer way was its chain of steps, not bytes: penalties 4.8
 // us, select 11.8 (four radix passes, a scan and a sort per slice), merge and
 // draw 14.6 (20 rounds of a 64-lane maximum, then one thread's loads from
-// LDS); now 5.3 and 11.2 us (248,320 logits, top 20, presence penalty over 1000
+// LDS); now 4.1 and 11.4 us (248,320 logits, top 20, presence penalty over 1000
 // ids).  The whole call in a replayed graph, us, longer / shorter way: spread
 // logits 28.8 / 14.5, sorted ones 29.0 / 22.6, all equal 30.3 / 26.8, all but
 // five masked 28.6 / 26.8; at top 64 57.3 / 25.4, 58.2 / 45.3, 60.8 / 48.7,
