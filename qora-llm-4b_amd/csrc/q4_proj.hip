@@ -81,8 +81,8 @@ QM_DEV void q4_accumulate(float (&acc)[8], uint32_t c, float sx) { q4_word(acc, 
 
 // Whether the wave's column sums are those of operands within the f16 codes'
 // range: one past it leaves every even column infinite or NaN, and the bits
-// lost to subnormals matter only where every sum is tiny.  Zeros are rows
-// past k.
+// lost to subnormals matter only where every sum is tiny (beside larger ones
+// they could break a rounding tie, no more).  Zeros are rows past k.
 QM_DEV bool q4_in_range(float y, float u) {
     constexpr uint32_t LO = 0x17800000u, INF = 0x7f800000u;   // 2^-80
     const uint32_t a = __float_as_uint(y) & 0x7fffffffu, b = __float_as_uint(u) & 0x7fffffffu, m = a > b ? a : b;
